@@ -512,3 +512,40 @@ def test_linear_matmul_override_on_gpu():
                        text=True, timeout=110)
     assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
     assert "override ok" in r.stdout
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 5, 31), (8, 4096, 256), (16, 17, 64), (17, 8197, 191),
+                                   (15, 30, 8200), (33, 100, 129), (64, 1000, 4161), (48, 63, 8192),
+                                   (64, 8192, 65)])
+@pytest.mark.parametrize("form", ["dense", "odd", "full_bias"])
+def test_few_rows_matmul(dtype, M, N, K, form):
+    """The few-row kernel (M <= 64) around its tiles (16 rows and columns, 64
+    k), its wave and K splits: dense operands, then rows at odd strides and
+    odd addresses with an odd-stride output, then a full fp32 bias with alpha
+    and beta."""
+    pad = 3 if form == "odd" else 0
+
+    def rows(r, c, seed):
+        t = rn((r * (c + pad) + 1,), seed, dtype, 1.0)
+        return t[1 if pad else 0:].narrow(0, 0, r * (c + pad)).view(r, c + pad)[:, :c]
+
+    a, b = rows(M, K, 60), rows(N, K, 61)
+    cuda = lambda t: torch.empty(t.untyped_storage().nbytes() // 2, dtype=dtype, device="cuda").copy_(
+        torch.tensor([], dtype=dtype).set_(t.untyped_storage())).as_strided(
+            t.shape, t.stride(), t.storage_offset())
+    out = torch.full((M, N + pad), 7.0, dtype=dtype, device="cuda")
+    o = out[:, :N]
+    if form == "full_bias":
+        bias = torch.randn(M, N, generator=g(62))
+        _abi.addmm(o, bias.cuda(), cuda(a), cuda(b).t(), beta=0.5, alpha=2.0)
+        ref = aten.addmm(bias, a, b.t(), beta=0.5, alpha=2.0)
+    elif form == "odd":
+        bias = rn((N,), 63, dtype, 1.0)
+        _abi.addmm(o, bias.cuda(), cuda(a), cuda(b).t())
+        ref = aten.addmm(bias, a, b.t())
+    else:
+        _abi.mm(o, cuda(a), cuda(b).t())
+        ref = aten.addmm(None, a, b.t(), beta=0.0)
+    assert_close(o, ref, "bf16", f"few rows {M}x{N}x{K} {form}")
+    assert bool((out[:, N:] == 7.0).all())  # nothing beyond the row

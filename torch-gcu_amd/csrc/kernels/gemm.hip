@@ -25,57 +25,13 @@
 // fp32 inputs take a VALU tiled kernel.
 #include <algorithm>
 
-#include "iter.h"
+#include "gemm_common.h"
 
 namespace mi {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr int BK = 64;
 constexpr int PITCH = BK + 8;  // LDS row pitch in elements
-
-template <typename T>
-struct MfmaOp;
-template <>
-struct MfmaOp<BF16> {
-  typedef bf16x8 vec;
-  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_bf16(v); }
-  static __device__ __forceinline__ float load(uint16_t v) { return bf16_to_f32(v); }
-};
-template <>
-struct MfmaOp<F16> {
-  typedef f16x8 vec;
-  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_f16(v); }
-  static __device__ __forceinline__ float load(uint16_t v) { return f16_to_f32(v); }
-};
-
-struct GemmArgs {
-  const uint16_t* a;  // [batch][M][lda], K contiguous
-  const void* b;      // [batch][N][ldb], K contiguous (16-bit or int8)
-  uint16_t* c;        // [batch][M][ldc], N contiguous
-  const void* bias;   // element (m, n) at bias + b*bias_sb + m*bias_sm + n*bias_sn
-  const float* scale; // int8 path: per-N fp32 scale
-  int bias_dtype;
-  int64_t bias_sm, bias_sn, bias_sb;
-  int64_t M, N, K;
-  int64_t lda, ldb, ldc;
-  int64_t sa, sb, sc;  // batch strides (elements)
-  float alpha, beta;
-  int tiles_m, tiles_n;
-  // fused epilogues of the large-tile kernel (EPI_SILU, EPI_RESID below)
-  const void* b2;       // EPI_SILU: the up weight, rows laid out like b's (the gate weight)
-  const uint16_t* res;  // EPI_RESID: residual, element (m, n) at res[m * ldr + n]
-  int64_t ldr;
-};
 
 __device__ __forceinline__ void tile_of(int bid, int tiles_m, int tiles_n, int* tm, int* tn) {
   const int total = tiles_m * tiles_n;
@@ -116,42 +72,6 @@ __device__ __forceinline__ typename MfmaOp<T>::vec widen8(u32x2_t w) {
       r[p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
   }
   return __builtin_bit_cast(typename MfmaOp<T>::vec, r);
-}
-
-
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
-
-// Four consecutive per-column values n .. n + 3 of a row vector (the int8
-// scale, or a bias broadcast over rows) as floats: element k at
-// base + off + k * stride, fp32 or of the output's 16-bit type T.  One
-// vector load when all four columns exist, the stride is 1 and the address
-// is aligned; else four loads with the column clamped to N - 1 (clamped
-// columns only feed outputs that are never stored).
-template <typename T>
-__device__ __forceinline__ f32x4_t load_col4_t(const void* base, int dtype, int64_t n, int64_t stride,
-                                               int64_t N, int64_t off) {
-  f32x4_t r;
-  if (dtype == MI_F32) {
-    const float* b = (const float*)base + off;
-    if (stride == 1 && n + 3 < N && (((uintptr_t)(b + n)) & 15) == 0) {
-      r = *(const f32x4_t*)(b + n);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) r[e] = b[min<int64_t>(n + e, N - 1) * stride];
-    }
-  } else {
-    const uint16_t* b = (const uint16_t*)base + off;
-    if (stride == 1 && n + 3 < N && (((uintptr_t)(b + n)) & 7) == 0) {
-      const u16x4_t v = *(const u16x4_t*)(b + n);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) r[e] = MfmaOp<T>::load(v[e]);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) r[e] = MfmaOp<T>::load(b[min<int64_t>(n + e, N - 1) * stride]);
-    }
-  }
-  return r;
 }
 
 // Per-lane loader of a ROWS x 64 tile of a K-contiguous 16-bit matrix: V
@@ -434,7 +354,6 @@ static_assert(LDS_BYTES8 <= 160 * 1024 && LDS_BYTES8 >= (size_t)NW * TM * EP * 2
 }  // namespace dl
 
 typedef __attribute__((address_space(3))) void lds_void_t;
-typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
 template <int N>
@@ -1216,7 +1135,6 @@ mi_status_t launch_mid(const GemmArgs& q0, hipStream_t s, const char* what) {
 // operands, so the sum is the plain dot product.  The 8 waves' partial
 // 16 x 16 tiles are added in a fixed order through LDS; the epilogue applies
 // the per-column scale and bias and rounds once.
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef int int4v_t __attribute__((ext_vector_type(4)));
 
 template <typename T>
@@ -2079,6 +1997,28 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
   // or B as row-major [K, N] rows read in place by the large-tile kernel
   Workspace wa, wb, wc;
   Mat Bt = transposed(B);
+  // few rows: the weight stream kernel, operands read as they are
+  if (!int8 && batch == 1 && M <= kRowsMax && (A.s1 == 1 || K == 1) && (Bt.s1 == 1 || K == 1) &&
+      (C.s1 == 1 || N == 1)) {
+    GemmArgs q{};
+    q.a = (const uint16_t*)A.data;
+    q.b = B.data;
+    q.c = (uint16_t*)C.data;
+    q.bias = bv.data;
+    q.bias_dtype = bv.dtype;
+    q.bias_sm = bv.sm;
+    q.bias_sn = bv.sn;
+    q.M = M;
+    q.N = N;
+    q.K = K;
+    q.lda = A.s0;
+    q.ldb = Bt.s0;
+    q.ldc = C.s0;
+    q.alpha = (float)alpha;
+    q.beta = (float)beta;
+    if (gemm_rows_eligible(q))
+      return launch_gemm_rows(q, A.dtype == MI_F16, has_bias, stream, what);
+  }
   MI_RETURN_IF(dense_rows(A, wa, stream));
   bool b_kn = false;
   if (!int8 && B.s1 == 1 && N > 1 && Bt.s1 != 1) {

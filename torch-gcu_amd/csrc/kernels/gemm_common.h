@@ -1,0 +1,98 @@
+// Types that the matrix-product kernels share: MFMA operand vectors, the
+// argument block and the per-column epilogue loads.
+#pragma once
+
+#include "iter.h"
+
+namespace mi {
+
+struct GemmArgs {
+  const uint16_t* a;  // [batch][M][lda], K contiguous
+  const void* b;      // [batch][N][ldb], K contiguous (16-bit or int8)
+  uint16_t* c;        // [batch][M][ldc], N contiguous
+  const void* bias;   // element (m, n) at bias + b*bias_sb + m*bias_sm + n*bias_sn
+  const float* scale; // int8 path: per-N fp32 scale
+  int bias_dtype;
+  int64_t bias_sm, bias_sn, bias_sb;
+  int64_t M, N, K;
+  int64_t lda, ldb, ldc;
+  int64_t sa, sb, sc;  // batch strides (elements)
+  float alpha, beta;
+  int tiles_m, tiles_n;
+  // fused epilogues of the large-tile kernel (EPI_SILU, EPI_RESID below)
+  const void* b2;       // EPI_SILU: the up weight, rows laid out like b's (the gate weight)
+  const uint16_t* res;  // EPI_RESID: residual, element (m, n) at res[m * ldr + n]
+  int64_t ldr;
+};
+
+// Few-row products (gemm_rows.hip): out = alpha * a b^T + beta * bias with
+// M <= kRowsMax, one batch, K-contiguous 16-bit operands of any alignment.
+constexpr int64_t kRowsMax = 64;
+bool gemm_rows_eligible(const GemmArgs& q);
+mi_status_t launch_gemm_rows(const GemmArgs& q, bool f16, bool has_bias, hipStream_t s,
+                             const char* what);
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <typename T>
+struct MfmaOp;
+template <>
+struct MfmaOp<BF16> {
+  typedef bf16x8 vec;
+  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_bf16(v); }
+  static __device__ __forceinline__ float load(uint16_t v) { return bf16_to_f32(v); }
+};
+template <>
+struct MfmaOp<F16> {
+  typedef f16x8 vec;
+  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint16_t store(float v) { return f32_to_f16(v); }
+  static __device__ __forceinline__ float load(uint16_t v) { return f16_to_f32(v); }
+};
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
+
+// Four consecutive per-column values n .. n + 3 of a row vector (the int8
+// scale, or a bias broadcast over rows) as floats: element k at
+// base + off + k * stride, fp32 or of the output's 16-bit type T.  One
+// vector load when all four columns exist, the stride is 1 and the address
+// is aligned; else four loads with the column clamped to N - 1 (clamped
+// columns only feed outputs that are never stored).
+template <typename T>
+__device__ __forceinline__ f32x4_t load_col4_t(const void* base, int dtype, int64_t n, int64_t stride,
+                                               int64_t N, int64_t off) {
+  f32x4_t r;
+  if (dtype == MI_F32) {
+    const float* b = (const float*)base + off;
+    if (stride == 1 && n + 3 < N && (((uintptr_t)(b + n)) & 15) == 0) {
+      r = *(const f32x4_t*)(b + n);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = b[min<int64_t>(n + e, N - 1) * stride];
+    }
+  } else {
+    const uint16_t* b = (const uint16_t*)base + off;
+    if (stride == 1 && n + 3 < N && (((uintptr_t)(b + n)) & 7) == 0) {
+      const u16x4_t v = *(const u16x4_t*)(b + n);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = MfmaOp<T>::load(v[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = MfmaOp<T>::load(b[min<int64_t>(n + e, N - 1) * stride]);
+    }
+  }
+  return r;
+}
+
+}  // namespace
+}  // namespace mi
