@@ -549,3 +549,34 @@ def test_few_rows_matmul(dtype, M, N, K, form):
         ref = aten.addmm(None, a, b.t(), beta=0.0)
     assert_close(o, ref, "bf16", f"few rows {M}x{N}x{K} {form}")
     assert bool((out[:, N:] == 7.0).all())  # nothing beyond the row
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 5), (65, 72, 63), (127, 129, 64), (128, 4096, 136),
+                                   (130, 70, 8191), (257, 255, 200), (300, 1000, 4161),
+                                   (777, 520, 2048), (1000, 2100, 320), (2050, 2049, 72)])
+@pytest.mark.parametrize("form", ["nk", "kn", "full_bias"])
+def test_middle_size_matmul(dtype, M, N, K, form):
+    """Products whose 256 x 256 tiles do not fill the CUs: every tile shape at
+    its edges, K slices, and K % 64 remainders (whole 16-byte chunks or not),
+    with a K-contiguous and a row-major B and a full bias."""
+    a, b = rn((M, K), 70, dtype, 1.0), rn((N, K), 71, dtype, 1.0)
+    bc = b.t().contiguous().cuda() if form == "kn" else b.cuda().t()
+    out = torch.empty(M, N, dtype=dtype, device="cuda")
+    if form == "full_bias":
+        bias = rn((M, N), 72, dtype, 1.0)
+        _abi.addmm(out, bias.cuda(), a.cuda(), bc, beta=0.5, alpha=2.0)
+        ref = aten.addmm(bias, a, b.t(), beta=0.5, alpha=2.0)
+    else:
+        _abi.mm(out, a.cuda(), bc)
+        ref = aten.addmm(None, a, b.t(), beta=0.0)
+    assert_close(out, ref, "bf16", f"middle {M}x{N}x{K} {form}")
+
+
+@pytest.mark.parametrize("Bt,M,N,K", [(64, 100, 100, 72), (7, 65, 33, 200), (3, 300, 260, 63)])
+def test_middle_size_bmm(Bt, M, N, K):
+    a, b = rn((Bt, M, K), 73, torch.bfloat16, 1.0), rn((Bt, K, N), 74, torch.bfloat16, 1.0)
+    out = torch.empty(Bt, M, N, dtype=torch.bfloat16, device="cuda")
+    _abi.bmm(out, a.cuda(), b.cuda())
+    assert_close(out, torch.stack([aten.addmm(None, x, y, beta=0.0) for x, y in zip(a, b)]), "bf16",
+                 f"bmm {Bt}x{M}x{N}x{K}")

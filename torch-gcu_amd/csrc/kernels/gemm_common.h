@@ -32,6 +32,16 @@ bool gemm_rows_eligible(const GemmArgs& q);
 mi_status_t launch_gemm_rows(const GemmArgs& q, bool f16, bool has_bias, hipStream_t s,
                              const char* what);
 
+// 16-bit products of any size by tile shape and K slices (gemm_mid.hip), for
+// operands with 16-byte aligned rows, K contiguous, and byte offsets below 4 GB.
+bool gemm_mid_eligible(const GemmArgs& q);
+mi_status_t launch_gemm_mid(const GemmArgs& q, int64_t batch, bool f16, bool has_bias,
+                            hipStream_t s, const char* what);
+// out = alpha * scale[n] * sum_s part[s] + beta * bias over S slices of raw
+// sums [M][ldp] (gemm.hip).
+mi_status_t launch_splitk_combine(const GemmArgs& q, bool f16, bool has_bias, const float* part,
+                                  int S, int64_t ldp, hipStream_t s, const char* what);
+
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -58,6 +68,30 @@ struct MfmaOp<F16> {
   static __device__ __forceinline__ uint16_t store(float v) { return f32_to_f16(v); }
   static __device__ __forceinline__ float load(uint16_t v) { return f16_to_f32(v); }
 };
+
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+// 8 int8 (two words) -> 8 x bf16 / f16, exact. One sign-extending byte
+// convert per value (v_cvt_f32_i32 with a byte select), then two values per
+// word: the upper halves of the two floats for bf16 (exact, an int8 has at
+// most 8 significant bits), a round-toward-zero pack for f16 (exact too).
+// 12 VALU per 8 values; a (__bf16) cast of the float costs twice that.
+template <typename T>
+__device__ __forceinline__ typename MfmaOp<T>::vec widen8(u32x2_t w) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 r;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const uint32_t d = w[p >> 1];
+    const float lo = (float)(int)(int8_t)(d >> (16 * (p & 1)));
+    const float hi = (float)(int)(int8_t)(d >> (16 * (p & 1) + 8));
+    if constexpr (std::is_same<T, BF16>::value)
+      r[p] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+    else
+      r[p] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+  }
+  return __builtin_bit_cast(typename MfmaOp<T>::vec, r);
+}
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
