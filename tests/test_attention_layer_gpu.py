@@ -345,3 +345,40 @@ def test_sdpa_grouped_query_heads_follow_enable_gqa():
     out2 = F.scaled_dot_product_attention(q2.to("gcu"), kb.to("gcu"), vb.to("gcu"))
     ref2 = F.scaled_dot_product_attention(q2.float(), kb.float(), vb.float())
     assert_close(out2.cpu(), ref2.to(torch.bfloat16), "bf16", "sdpa broadcast batch")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,Hk,Sq,Sk,D", [
+    (1, 1, 1, 1, 1001, 128),   # keys split, the last tile of 9 keys
+    (2, 8, 2, 1, 4096, 64),
+    (1, 32, 1, 1, 2047, 128),  # 32 rows, one tile exactly
+    (3, 16, 4, 8, 700, 128),   # 32 rows over four heads and eight queries
+    (1, 8, 1, 5, 513, 64),     # 40 rows: a second, partial row tile
+    (65, 8, 4, 2, 225, 128),   # heads enough for the CUs: no key split
+])
+@pytest.mark.parametrize("form", ["dense", "heads_inner", "negative_scale", "ramp"])
+def test_attention_few_queries_long_cache(dtype, B, H, Hk, Sq, Sk, D, form):
+    """The key-split kernel: row tiles, key remainders, grouped heads and both
+    layouts, a negative scale and scores that grow along the keys (so every
+    wave and split has its own max to merge)."""
+    q, k, v = rn((B, H, Sq, D), 81, dtype), rn((B, Hk, Sk, D), 82, dtype), rn((B, Hk, Sk, D), 83, dtype)
+    if form == "ramp":
+        k = (k.float() * torch.linspace(0.2, 4.0, Sk)[None, None, :, None]).to(dtype)
+    if form == "negative_scale":
+        scale = -0.07
+        kk, vv = (t.repeat_interleave(H // Hk, 1).float().numpy() for t in (k, v))
+        ro, rl = npr.attention64(q.float().numpy(), kk, vv, False, scale)
+        ref, ref_lse = torch.from_numpy(ro).to(dtype), torch.from_numpy(rl).float()
+    else:
+        scale = None
+        ref, ref_lse = ref_attention(q, k, v, False)
+    if form == "heads_inner":
+        dev = [t.transpose(1, 2).contiguous().cuda().transpose(1, 2) for t in (q, k, v)]
+        out = torch.empty(B, Sq, H, D, dtype=dtype, device="cuda").transpose(1, 2)
+    else:
+        dev = [t.cuda() for t in (q, k, v)]
+        out = torch.empty(B, H, Sq, D, dtype=dtype, device="cuda")
+    lse = torch.empty(B, H, Sq, dtype=torch.float32, device="cuda")
+    _abi.flash_attention_fwd(out, lse, *dev, False, scale)
+    assert_close(out, ref, "bf16", f"few queries {B},{H},{Hk},{Sq},{Sk},{D} {form}")
+    assert (lse.cpu() - ref_lse).abs().max().item() < 2e-2 * max(1.0, ref_lse.abs().max().item())

@@ -32,57 +32,10 @@
 // the 8 XCDs (which receive workgroups round robin) walks a contiguous run of
 // heads: a head's K/V is then read into one XCD's L2 while its query tiles
 // run there.
-#include <cmath>
-
-#include "iter.h"
+#include "attention_common.h"
 
 namespace mi {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-template <typename T>
-struct AttnOp;
-template <>
-struct AttnOp<BF16> {
-  typedef bf16x8 vec;
-  typedef __bf16 elem;
-  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
-};
-template <>
-struct AttnOp<F16> {
-  typedef f16x8 vec;
-  typedef _Float16 elem;
-  static __device__ __forceinline__ f32x16 mma(vec a, vec b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-struct AttnArgs {
-  const uint16_t* q;
-  const uint16_t* k;
-  const uint16_t* v;
-  uint16_t* o;
-  float* lse;
-  int64_t H, Hk, Sq, Sk;
-  int64_t q_sb, q_sh, q_ss;
-  int64_t k_sb, k_sh, k_ss;
-  int64_t v_sb, v_sh, v_ss;
-  int64_t o_sb, o_sh, o_ss;
-  int64_t lse_sb, lse_sh;
-  float scale_log2;  // softmax scale * log2(e)
-  int causal;
-  int q_tiles;
-  int n_blocks;      // q_tiles * H * B
-  int xcd_remap;     // n_blocks % 8 == 0: renumber blocks per XCD
-};
 
 constexpr int QT = 128;  // query rows per block
 constexpr int KT = 64;   // keys per tile
@@ -107,8 +60,8 @@ struct FlashCfg {
   static constexpr int NINS = KT / RPI; // wave copies per K (or V) tile
   static constexpr int TILE = KT * D;   // elements of one K (or V) tile
   static constexpr int STAGE = 2 * TILE;
-  static __device__ __forceinline__ int swz_k(int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); }
-  static __device__ __forceinline__ int swz_v(int r) { return D == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); }
+  static __device__ __forceinline__ int swz_k(int r) { return swz_k_of<D>(r); }
+  static __device__ __forceinline__ int swz_v(int r) { return swz_v_of<D>(r); }
   static_assert(NINS % 4 == 0, "four waves share a tile's copies");
 };
 
@@ -590,6 +543,8 @@ extern "C" mi_status_t mi_flash_attention_fwd(const mi_tensor_t* out, const mi_t
   a.n_blocks = (int)nb;
   a.xcd_remap = (nb % 8 == 0) ? 1 : 0;
   hipStream_t s = (hipStream_t)stream;
+  mi_status_t st;
+  if (flash_decode(a, B, D, q->dtype == MI_F16, s, &st)) return st;
   if (q->dtype == MI_BF16)
     return D == 128 ? launch_flash<BF16, 128>(a, s) : launch_flash<BF16, 64>(a, s);
   return D == 128 ? launch_flash<F16, 128>(a, s) : launch_flash<F16, 64>(a, s);
