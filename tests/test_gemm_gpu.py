@@ -580,3 +580,40 @@ def test_middle_size_bmm(Bt, M, N, K):
     _abi.bmm(out, a.cuda(), b.cuda())
     assert_close(out, torch.stack([aten.addmm(None, x, y, beta=0.0) for x, y in zip(a, b)]), "bf16",
                  f"bmm {Bt}x{M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (3, 200, 33), (42, 1216, 768), (65, 63, 31), (64, 64, 4100),
+                                   (130, 257, 100), (2000, 2048, 96), (1030, 1025, 65)])
+@pytest.mark.parametrize("lay", ["nn", "nt", "tn", "tt", "odd"])
+def test_f32_matmul_layouts(M, N, K, lay):
+    """The fp32 kernel in every operand layout (contiguous along K or along
+    the rows, and neither), at tile edges, K remainders and K slices, with and
+    without a bias, against float64 (bound: K/2 ulp of the sum of magnitudes
+    would be 6e-8 K; the fp32 bar covers the random sums here)."""
+    a, b = torch.randn(M, K, generator=g(80)), torch.randn(K, N, generator=g(81))
+    if lay == "odd":  # every second column of a wider matrix, rows at an odd stride
+        wide = torch.randn(M, 2 * K + 1, generator=g(82))
+        a = wide[:, ::2][:, :K]
+        da = wide.cuda()[:, ::2][:, :K]
+        db = torch.randn(2 * N + 1, K + 3, generator=g(83))
+        b = db[::2, 1:K + 1][:N].t()
+        db = db.cuda()[::2, 1:K + 1][:N].t()
+    else:
+        da = a.cuda() if lay[0] == "n" else a.t().contiguous().cuda().t()
+        db = b.cuda() if lay[1] == "n" else b.t().contiguous().cuda().t()
+    out = torch.full((M, N + 1), 7.0, device="cuda")
+    ref = a.double() @ b.double()
+    _abi.mm(out[:, :N], da, db)
+    assert_close(out[:, :N], ref.float(), "fp32", f"f32 mm {M}x{N}x{K} {lay}")
+    bias = torch.randn(N, generator=g(84))
+    _abi.addmm(out[:, :N], bias.cuda(), da, db, beta=0.5, alpha=2.0)
+    assert_close(out[:, :N], (2 * ref + 0.5 * bias.double()).float(), "fp32", f"f32 addmm {lay}")
+    assert bool((out[:, N] == 7.0).all())
+
+
+def test_f32_bmm_layouts():
+    a, b = torch.randn(5, 70, 200, generator=g(85)), torch.randn(5, 200, 33, generator=g(86))
+    out = torch.empty(5, 70, 33, device="cuda")
+    for bb in (b.cuda(), b.transpose(1, 2).contiguous().cuda().transpose(1, 2)):
+        _abi.bmm(out, a.cuda(), bb)
+        assert_close(out, torch.bmm(a.double(), b.double()).float(), "fp32", "f32 bmm")

@@ -26,10 +26,11 @@
 // Workgroups are renumbered so that each of the 8 XCDs (which receive
 // workgroups round robin) gets a contiguous run of tiles, walked in groups
 // of 8 row panels, so tiles sharing A and B panels meet in one L2.
-// fp32 inputs take a VALU tiled kernel.
+// fp32 inputs run gemm_f32.hip.
 #include <algorithm>
 
 #include "gemm_dl.h"
+#include "gemm_f32.h"
 
 namespace mi {
 namespace {
@@ -925,72 +926,6 @@ mi_status_t launch_stream(const GemmArgs& q, hipStream_t s) {
   }
 }
 
-// ---- fp32: VALU tiled kernel (64 x 64 tile, 4 x 4 outputs per lane) ----------------
-
-struct GemmF32Args {
-  const float* a;
-  const float* b;
-  float* c;
-  const void* bias;
-  int bias_dtype;
-  int64_t bias_sm, bias_sn, bias_sb;
-  int64_t M, N, K;
-  int64_t a_sm, a_sk, b_sk, b_sn, ldc;
-  int64_t sa, sb, sc;
-  float alpha, beta;
-};
-
-template <bool HAS_BIAS>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args p) {
-  __shared__ float As[16][64 + 4];
-  __shared__ float Bs[16][64 + 4];
-  const int64_t batch = blockIdx.z;
-  const float* A = p.a + batch * p.sa;
-  const float* B = p.b + batch * p.sb;
-  const int64_t m0 = (int64_t)blockIdx.y * 64, n0 = (int64_t)blockIdx.x * 64;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  float acc[4][4] = {};
-  for (int64_t k0 = 0; k0 < p.K; k0 += 16) {
-    for (int v = threadIdx.x; v < 16 * 64; v += 256) {
-      const int kk = v / 64, mm = v % 64;
-      const int64_t gm = m0 + mm, gk = k0 + kk;
-      As[kk][mm] = (gm < p.M && gk < p.K) ? A[gm * p.a_sm + gk * p.a_sk] : 0.f;
-      const int64_t gn = n0 + mm;
-      Bs[kk][mm] = (gn < p.N && gk < p.K) ? B[gk * p.b_sk + gn * p.b_sn] : 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-  float* C = p.c + batch * p.sc;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t m = m0 + ty * 4 + i;
-    if (m >= p.M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t n = n0 + tx * 4 + j;
-      if (n >= p.N) continue;
-      float v = p.alpha * acc[i][j];
-      if (HAS_BIAS)
-        v += p.beta * load_as<float>(p.bias, batch * p.bias_sb + m * p.bias_sm + n * p.bias_sn,
-                                     p.bias_dtype);
-      C[m * p.ldc + n] = v;
-    }
-  }
-}
-
 // ---- host side --------------------------------------------------------------------
 
 // A batched matrix view: element (b, r, c) at data + b*sb + r*s0 + c*s1.
@@ -1428,10 +1363,7 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
     q.sc = C.sb;
     q.alpha = (float)alpha;
     q.beta = (float)beta;
-    dim3 grid(ceil_div_u(N, 64), ceil_div_u(M, 64), (unsigned)batch);
-    if (has_bias) hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, dim3(256), 0, stream, q);
-    else hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, dim3(256), 0, stream, q);
-    return check_launch(what);
+    return launch_gemm_f32(q, batch, has_bias, stream, what);
   }
 
   // MFMA path: A as [M, K] rows, B as [N, K] rows (B^T with K contiguous),
