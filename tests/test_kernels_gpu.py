@@ -728,3 +728,60 @@ def test_backward_ops_abi(dtype):
     # only the column sums, no weight
     _abi.layer_norm_backward(None, None, db, dev(dy), dev(x), dev(mean), dev(rstd), None, 1024)
     assert_close(db, torch.from_numpy(rdb).to(dtype), kind, "layer_norm dbeta alone")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("width", [1, 3, 9, 511, 513, 1025, 2047, 4099, 8200, 32001, 50257, 65543, 131075,
+                                   140001])
+def test_rows_at_any_offset(width, dtype):
+    """log_softmax, its backward, sum and amax over rows that start at every
+    element offset (odd widths behind an odd base) and over rows longer than
+    the register kernels hold; one row all -inf but its last element."""
+    rows = 5 if width > 1000 else 131
+    gen = torch.Generator().manual_seed(width)
+
+    def odd(t):  # the same values behind one extra element
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+        buf[1:].copy_(t.reshape(-1))
+        return buf[1:].view(t.shape)
+
+    x = (torch.randn(rows, width, generator=gen) * 4).to(dtype)
+    x[1, :-1] = -float("inf")
+    kind = "fp32" if dtype == torch.float32 else "bf16"
+    y = aten.log_softmax(x, -1)
+    out = odd(torch.zeros_like(x))
+    _abi.log_softmax(out, odd(x), -1)
+    fin = torch.isfinite(y)
+    assert torch.equal(torch.isfinite(out.cpu()), fin)
+    assert_close(out.cpu()[fin], y[fin], kind, f"log_softmax {width}")
+    sm = odd(torch.zeros_like(x))
+    _abi.softmax(sm, odd(x), -1)
+    assert_close(sm, aten.softmax(x, -1), kind, f"softmax {width}")
+    x[1] = 0
+    y = aten.log_softmax(x, -1)
+    dy = torch.randn(rows, width, generator=gen).to(dtype)
+    gi = odd(torch.zeros_like(x))
+    _abi.log_softmax_backward(gi, odd(dy), odd(y), -1)
+    assert_close(gi, aten.log_softmax_backward(dy, y, -1, dtype), kind, f"backward {width}")
+    s, m = torch.empty(rows, dtype=dtype, device="cuda"), torch.empty(rows, dtype=dtype, device="cuda")
+    _abi.sum_(s, odd(x), [-1])
+    assert_close(s, aten.sum_(x, -1), kind, f"sum {width}")
+    _abi.amax(m, odd(x), [-1])
+    assert_exact(m, aten.amax(x, -1), f"amax {width}")
+
+
+@pytest.mark.parametrize("dtype", [torch.int8, torch.int32, torch.int64, torch.float64])
+def test_row_reductions_of_short_rows_at_any_offset(dtype):
+    gen = torch.Generator().manual_seed(3)
+    for rows, width in [(300, 77), (2100, 2049), (3, 4097)]:
+        x = torch.randint(-9, 9, (rows, width), generator=gen).to(dtype)
+        buf = torch.empty(x.numel() + 1, dtype=dtype, device="cuda")
+        buf[1:].copy_(x.reshape(-1))
+        xd = buf[1:].view(rows, width)
+        m = torch.empty(rows, dtype=dtype, device="cuda")
+        _abi.amax(m, xd, [-1])
+        assert_exact(m, x.amax(-1), f"amax {rows}x{width}")
+        sd = torch.float64 if dtype == torch.float64 else torch.int64
+        s = torch.empty(rows, dtype=sd, device="cuda")
+        _abi.sum_(s, xd, [-1])
+        assert_exact(s, x.sum(-1, dtype=sd), f"sum {rows}x{width}")

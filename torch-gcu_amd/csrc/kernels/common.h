@@ -397,6 +397,38 @@ __device__ __forceinline__ void st_stream(V* p, const V& v) {
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), (u32x4_t*)p);
 }
 
+// The same from / to any address that is a multiple of the element S: global
+// 16-byte accesses may start at any byte, so a row at an odd offset (a 50257-wide
+// vocabulary) keeps them and pays only for the lines its lanes straddle.
+template <int N>
+struct AnyAligned;
+template <>
+struct AnyAligned<1> {
+  typedef u32x4_t __attribute__((aligned(1))) type;
+};
+template <>
+struct AnyAligned<2> {
+  typedef u32x4_t __attribute__((aligned(2))) type;
+};
+template <>
+struct AnyAligned<4> {
+  typedef u32x4_t __attribute__((aligned(4))) type;
+};
+template <>
+struct AnyAligned<8> {
+  typedef u32x4_t __attribute__((aligned(8))) type;
+};
+template <typename S, typename V>
+__device__ __forceinline__ V ld_stream_any(const void* p) {
+  static_assert(sizeof(V) == 16, "16-byte type expected");
+  return __builtin_bit_cast(V, __builtin_nontemporal_load((const typename AnyAligned<sizeof(S)>::type*)p));
+}
+template <typename S, typename V>
+__device__ __forceinline__ void st_stream_any(void* p, const V& v) {
+  static_assert(sizeof(V) == 16, "16-byte type expected");
+  __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, v), (typename AnyAligned<sizeof(S)>::type*)p);
+}
+
 inline unsigned ceil_div_u(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
 }  // namespace mi

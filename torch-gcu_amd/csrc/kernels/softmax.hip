@@ -7,8 +7,11 @@
 //   log_softmax: x - max - log(sum)      softmax: exp(x - max) * (1 / sum)
 // which is the same sequence of float operations ATen's CPU kernel uses
 // (aten/src/ATen/native/cpu/SoftMaxKernel.cpp, _vec_log_softmax_lastdim).
-// Longer or unaligned rows use a two-read block kernel with an online
-// (max, sum) pair; a non-last dim uses one lane per column.
+// Rows at any element offset and of any length take the same kernel with
+// 16-byte accesses at element alignment and the last D % VEC elements one per
+// lane (ANY; bf16 [2048, 50257]: 217 us in scalar loads before, backward 250).
+// Longer rows use a two-read block kernel with an online (max, sum) pair; a
+// non-last dim uses one lane per column.
 #include <cmath>
 
 #include "iter.h"
@@ -45,28 +48,6 @@ __device__ __forceinline__ float kexp(float x) {
   else return fast_exp(x);
 }
 
-__device__ __forceinline__ float block_max_f(float v, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  v = wave_nan_max(v);
-  if (lane == 0) red[wid] = v;
-  __syncthreads();
-  float r = red[0];
-  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) r = nan_max(r, red[w]);
-  __syncthreads();
-  return r;
-}
-
-__device__ __forceinline__ float block_sum_f(float v, float* red) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  v = wave_sum(v);
-  if (lane == 0) red[wid] = v;
-  __syncthreads();
-  float r = red[0];
-  for (int w = 1; w < (int)(blockDim.x >> 6); ++w) r += red[w];
-  __syncthreads();
-  return r;
-}
-
 // Register-resident row: NTH lanes, VPT 16-byte vectors per lane.  The row
 // max uses fmaxf, which skips NaN: a NaN element still makes exp(x - max)
 // and therefore the row sum NaN, so every output of that row is NaN, as in
@@ -76,6 +57,7 @@ template <int NTH>
 __device__ __forceinline__ float block_fmax(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   v = wave_fmax(v);
+  if constexpr (NTH == 64) return v;
   if (lane == 0) red[wid] = v;
   __syncthreads();
   float r = red[0];
@@ -87,6 +69,7 @@ template <int NTH>
 __device__ __forceinline__ float block_fsum(float v, float* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   v = wave_sum(v);
+  if constexpr (NTH == 64) return v;
   if (lane == 0) red[wid] = v;
   __syncthreads();
   float r = red[0];
@@ -95,11 +78,21 @@ __device__ __forceinline__ float block_fsum(float v, float* red) {
   return r;
 }
 
-template <typename InTag, typename OutTag, int NTH, int VPT, bool LOG>
-__global__ __launch_bounds__(NTH) void softmax_reg_kernel(
+// NTH = 64: a wave per row, four rows per block (64 x 4 lanes), no barrier; for
+// short rows a block per row is all launch and reduction (log_softmax bf16
+// [20000, 500] 18.2 us with 256 lanes a row, 9.4 so; backward 16.5 and 12.7).
+// Up to 128 vectors a row: at 250 (bf16 [8192, 2000]) the forward ties, the
+// backward takes 19.4 us against 17.7, and few rows are slower.
+template <int NTH>
+__device__ __forceinline__ int64_t reg_row() {
+  return NTH == 64 ? (int64_t)blockIdx.x * 4 + threadIdx.y : (int64_t)blockIdx.x;
+}
+
+template <typename InTag, typename OutTag, int NTH, int VPT, bool LOG, bool ANY>
+__global__ __launch_bounds__(NTH == 64 ? 256 : NTH) void softmax_reg_kernel(
     typename ST<OutTag>::storage* __restrict__ out,
-    const typename ST<InTag>::storage* __restrict__ in, int64_t D, int64_t in_row_stride,
-    int64_t out_row_stride) {
+    const typename ST<InTag>::storage* __restrict__ in, int64_t rows, int64_t D,
+    int64_t in_row_stride, int64_t out_row_stride) {
   typedef typename ST<InTag>::storage Si;
   typedef typename ST<OutTag>::storage So;
   constexpr int VEC = 16 / sizeof(Si);
@@ -113,16 +106,28 @@ __global__ __launch_bounds__(NTH) void softmax_reg_kernel(
     So s[VEC];
     uint4 u[kWords];
   };
-  const int64_t row = blockIdx.x;
+  const int64_t row = reg_row<NTH>();
+  if (NTH == 64 && row >= rows) return;
   const Vi* pin = (const Vi*)(in + row * in_row_stride);
   const int nv = (int)(D / VEC);
+  // ANY: lane t < D % VEC holds element nv VEC + t too
+  const bool rem = ANY && (int)threadIdx.x < (int)(D - (int64_t)nv * VEC);
+  float xr = -INFINITY;
+  if constexpr (ANY) {
+    const Si* pr = in + row * in_row_stride;
+    xr = ST<InTag>::load(pr[rem ? (int64_t)nv * VEC + threadIdx.x : D - 1]);
+  }
   Vi x[VPT];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int v = threadIdx.x + k * NTH;
-    if (v < nv) x[k] = ld_stream(pin + v);
+    if constexpr (ANY) {
+      if (v < nv) x[k] = ld_stream_any<Si, Vi>((const Si*)pin + (int64_t)v * VEC);
+    } else {
+      if (v < nv) x[k] = ld_stream(pin + v);
+    }
   }
-  float m = -INFINITY;
+  float m = rem ? xr : -INFINITY;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     if ((int)threadIdx.x + k * NTH < nv) {
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(NTH) void softmax_reg_kernel(
     }
   }
   m = block_fmax<NTH>(m, red[0]);
-  float s = 0.f;
+  float s = rem ? kexp<InTag>(xr - m) : 0.f;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     if ((int)threadIdx.x + k * NTH < nv) {
@@ -152,9 +157,13 @@ __global__ __launch_bounds__(NTH) void softmax_reg_kernel(
         for (int e = 0; e < VEC; ++e)
           o.s[e] = ST<OutTag>::store((ST<InTag>::load(x[k].s[e]) - m) - lse);
 #pragma unroll
-        for (int w = 0; w < kWords; ++w) st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        for (int w = 0; w < kWords; ++w) {
+          if constexpr (ANY) st_stream_any<So>((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+          else st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        }
       }
     }
+    if (rem) po[(int64_t)nv * VEC + threadIdx.x] = ST<OutTag>::store((xr - m) - lse);
   } else {
     const float inv = 1.0f / s;
 #pragma unroll
@@ -166,50 +175,93 @@ __global__ __launch_bounds__(NTH) void softmax_reg_kernel(
         for (int e = 0; e < VEC; ++e)
           o.s[e] = ST<OutTag>::store(kexp<InTag>(ST<InTag>::load(x[k].s[e]) - m) * inv);
 #pragma unroll
-        for (int w = 0; w < kWords; ++w) st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        for (int w = 0; w < kWords; ++w) {
+          if constexpr (ANY) st_stream_any<So>((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+          else st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        }
       }
     }
+    if (rem) po[(int64_t)nv * VEC + threadIdx.x] = ST<OutTag>::store(kexp<InTag>(xr - m) * inv);
   }
 }
 
-// Any row length / alignment: online (max, sum) in one read, output in a
-// second read.
+// Rows longer than the registers: 1024 lanes, an online (max, sum) in one read
+// of four 16-byte vectors per lane at a time, the output in a second read.  A
+// lane whose elements were all -inf (or NaN) keeps max -inf and sum 0 (or NaN).
+constexpr int kLong = 1024, kLongU = 4;
 template <typename InTag, typename OutTag, bool LOG>
-__global__ __launch_bounds__(kBlock) void softmax_row_kernel(
+__global__ __launch_bounds__(kLong) void softmax_row_kernel(
     typename ST<OutTag>::storage* __restrict__ out,
     const typename ST<InTag>::storage* __restrict__ in, int64_t D, int64_t in_row_stride,
     int64_t out_row_stride) {
-  __shared__ float red[16];
-  __shared__ float red2[16];
+  typedef typename ST<InTag>::storage Si;
+  typedef typename ST<OutTag>::storage So;
+  constexpr int VEC = 16 / sizeof(Si), kWords = sizeof(So) * VEC / 16;
+  __shared__ float red[2][kLong / 64];
+  union Vi {
+    uint4 u;
+    Si s[VEC];
+  };
+  union Vo {
+    So s[VEC];
+    uint4 u[kWords];
+  };
   const int64_t row = blockIdx.x;
-  const typename ST<InTag>::storage* p = in + row * in_row_stride;
+  const Si* p = in + row * in_row_stride;
+  So* po = out + row * out_row_stride;
+  const int64_t nv = D / VEC, tail = nv * VEC + threadIdx.x;
   float m = -INFINITY, s = 0.f;
-  for (int64_t j = threadIdx.x; j < D; j += kBlock) {
-    const float x = ST<InTag>::load(p[j]);
-    if (x != x) {
-      m = x;  // NaN propagates through max and sum
-    } else if (x > m) {
-      s = s * kexp<InTag>(m - x) + 1.f;
-      m = x;
-    } else if (x > -INFINITY) {
-      s += kexp<InTag>(x - m);
+  auto load = [&](Vi* x, int64_t v0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)
+      x[u] = ld_stream_any<Si, Vi>(p + min(v0 + (int64_t)u * kLong, nv - 1) * VEC);
+  };
+  for (int64_t v0 = threadIdx.x; v0 < nv; v0 += kLong * kLongU) {
+    Vi x[kLongU];
+    load(x, v0);
+    float mn = m;
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)
+      if (v0 + (int64_t)u * kLong < nv)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) mn = fmaxf(mn, ST<InTag>::load(x[u].s[e]));
+    const float mu = mn == -INFINITY ? 0.f : mn;
+    s *= m == -INFINITY ? 1.f : kexp<InTag>(m - mu);
+    m = mn;
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)
+      if (v0 + (int64_t)u * kLong < nv)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s += kexp<InTag>(ST<InTag>::load(x[u].s[e]) - mu);
+  }
+  if (tail < D) {
+    const float x = ST<InTag>::load(p[tail]), mn = fmaxf(m, x), mu = mn == -INFINITY ? 0.f : mn;
+    s = s * (m == -INFINITY ? 1.f : kexp<InTag>(m - mu)) + kexp<InTag>(x - mu);
+    m = mn;
+  }
+  const float gm = block_fmax<kLong>(m, red[0]);
+  const float gs =
+      block_fsum<kLong>(s * (m == -INFINITY ? 1.f : kexp<InTag>(m - gm)), red[1]);
+  const float lse = LOG ? logf(gs) : 0.f, inv = 1.0f / gs;
+  auto value = [&](float x) __attribute__((always_inline)) {
+    return ST<OutTag>::store(LOG ? (x - gm) - lse : kexp<InTag>(x - gm) * inv);
+  };
+  for (int64_t v0 = threadIdx.x; v0 < nv; v0 += kLong * kLongU) {
+    Vi x[kLongU];
+    load(x, v0);
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u) {
+      const int64_t v = v0 + (int64_t)u * kLong;
+      if (v < nv) {
+        Vo o;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) o.s[e] = value(ST<InTag>::load(x[u].s[e]));
+#pragma unroll
+        for (int w = 0; w < kWords; ++w) st_stream_any<So>((uint4*)(po + v * VEC) + w, o.u[w]);
+      }
     }
   }
-  // combine (m, s) pairs across the block
-  const float gm = block_max_f(m, red);
-  float ls = (m == -INFINITY) ? 0.f : s * kexp<InTag>(m - gm);
-  (void)red2;
-  const float gs = block_sum_f(ls, red);
-  typename ST<OutTag>::storage* po = out + row * out_row_stride;
-  if constexpr (LOG) {
-    const float lse = logf(gs);
-    for (int64_t j = threadIdx.x; j < D; j += kBlock)
-      po[j] = ST<OutTag>::store((ST<InTag>::load(p[j]) - gm) - lse);
-  } else {
-    const float inv = 1.0f / gs;
-    for (int64_t j = threadIdx.x; j < D; j += kBlock)
-      po[j] = ST<OutTag>::store(kexp<InTag>(ST<InTag>::load(p[j]) - gm) * inv);
-  }
+  if (tail < D) po[tail] = value(ST<InTag>::load(p[tail]));
 }
 
 // [outer, D, inner] with inner > 1: one lane per (outer, inner) column.
@@ -256,17 +308,25 @@ mi_status_t launch_t(const mi_tensor_t* out, const mi_tensor_t* self, int dim,
     auto run_reg = [&](auto nth_c, auto vpt_c) -> mi_status_t {
       constexpr int NTH = decltype(nth_c)::value;
       constexpr int VPT = decltype(vpt_c)::value;
-      hipLaunchKernelGGL((softmax_reg_kernel<InTag, OutTag, NTH, VPT, LOG>),
-                         dim3((unsigned)outer), dim3(NTH), 0, stream,
-                         (typename ST<OutTag>::storage*)out->data, (const Si*)self->data, D, D,
-                         D);
+      const dim3 grid((unsigned)(NTH == 64 ? (outer + 3) / 4 : outer)), block(NTH, NTH == 64 ? 4 : 1);
+      if (aligned)
+        hipLaunchKernelGGL((softmax_reg_kernel<InTag, OutTag, NTH, VPT, LOG, false>), grid, block, 0,
+                           stream, (typename ST<OutTag>::storage*)out->data,
+                           (const Si*)self->data, outer, D, D, D);
+      else
+        hipLaunchKernelGGL((softmax_reg_kernel<InTag, OutTag, NTH, VPT, LOG, true>), grid, block, 0,
+                           stream, (typename ST<OutTag>::storage*)out->data,
+                           (const Si*)self->data, outer, D, D, D);
       return check_launch("softmax_reg");
     };
     typedef std::integral_constant<int, 1> V1;
+    typedef std::integral_constant<int, 64> N64;
     typedef std::integral_constant<int, 1024> N1024;
     // rows of up to 256 K vectors: 1024 lanes hold up to 16 vectors each
     // (64 VGPRs of row data); short rows take one vector per lane
-    if (aligned && nv <= 1024 * 16 && outer <= 0x7fffffff) {
+    if (nv <= 1024 * 16 && outer <= 0x7fffffff) {
+      if (nv <= 64) return run_reg(N64(), V1());
+      if (nv <= 128) return run_reg(N64(), std::integral_constant<int, 2>());
       if (nv <= 256) return run_reg(std::integral_constant<int, 256>(), V1());
       if (nv <= 512) return run_reg(std::integral_constant<int, 512>(), V1());
       if (nv <= 1024) return run_reg(N1024(), V1());
@@ -276,7 +336,7 @@ mi_status_t launch_t(const mi_tensor_t* out, const mi_tensor_t* self, int dim,
       return run_reg(N1024(), std::integral_constant<int, 16>());
     }
     hipLaunchKernelGGL((softmax_row_kernel<InTag, OutTag, LOG>), dim3((unsigned)outer),
-                       dim3(kBlock), 0, stream, (typename ST<OutTag>::storage*)out->data,
+                       dim3(kLong), 0, stream, (typename ST<OutTag>::storage*)out->data,
                        (const Si*)self->data, D, D, D);
     return check_launch("softmax_row");
   }
@@ -304,10 +364,10 @@ __device__ __forceinline__ float bwd_out(float dy, float y, float s) {
   else return y * (dy - s);
 }
 
-template <typename InTag, typename OutTag, int NTH, int VPT, bool LOG>
-__global__ __launch_bounds__(NTH) void softmax_bwd_reg_kernel(
+template <typename InTag, typename OutTag, int NTH, int VPT, bool LOG, bool ANY>
+__global__ __launch_bounds__(NTH == 64 ? 256 : NTH) void softmax_bwd_reg_kernel(
     typename ST<OutTag>::storage* __restrict__ gi, const typename ST<InTag>::storage* __restrict__ dy,
-    const typename ST<InTag>::storage* __restrict__ y, int64_t D) {
+    const typename ST<InTag>::storage* __restrict__ y, int64_t rows, int64_t D) {
   typedef typename ST<InTag>::storage Si;
   typedef typename ST<OutTag>::storage So;
   constexpr int VEC = 16 / sizeof(Si);
@@ -324,20 +384,34 @@ __global__ __launch_bounds__(NTH) void softmax_bwd_reg_kernel(
     uint2 h[kBytes / 8];
     uint4 u[(kBytes + 15) / 16];
   };
-  const int64_t row = blockIdx.x;
+  const int64_t row = reg_row<NTH>();
+  if (NTH == 64 && row >= rows) return;
   const Vi* pd = (const Vi*)(dy + row * D);
   const Vi* py = (const Vi*)(y + row * D);
   const int nv = (int)(D / VEC);
+  // ANY: lane t < D % VEC holds element nv VEC + t too
+  const bool rem = ANY && (int)threadIdx.x < (int)(D - (int64_t)nv * VEC);
+  const int64_t tail = rem ? (int64_t)nv * VEC + threadIdx.x : D - 1;
+  float rd = 0.f, ry = 0.f;
+  if constexpr (ANY) {
+    rd = ST<InTag>::load(((const Si*)pd)[tail]);
+    ry = ST<InTag>::load(((const Si*)py)[tail]);
+  }
   Vi xd[VPT], xy[VPT];
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int v = threadIdx.x + k * NTH;
     if (v < nv) {
-      xd[k] = ld_stream(pd + v);
-      xy[k] = ld_stream(py + v);
+      if constexpr (ANY) {
+        xd[k] = ld_stream_any<Si, Vi>((const Si*)pd + (int64_t)v * VEC);
+        xy[k] = ld_stream_any<Si, Vi>((const Si*)py + (int64_t)v * VEC);
+      } else {
+        xd[k] = ld_stream(pd + v);
+        xy[k] = ld_stream(py + v);
+      }
     }
   }
-  float s = 0.f;
+  float s = rem ? bwd_term<InTag, LOG>(rd, ry) : 0.f;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     if ((int)threadIdx.x + k * NTH < nv) {
@@ -358,30 +432,80 @@ __global__ __launch_bounds__(NTH) void softmax_bwd_reg_kernel(
         o.s[e] = ST<OutTag>::store(
             bwd_out<InTag, LOG>(ST<InTag>::load(xd[k].s[e]), ST<InTag>::load(xy[k].s[e]), s));
       if constexpr (kBytes == 8) {
-        *(uint2*)(po + (int64_t)v * VEC) = o.h[0];
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        typedef u32x2 __attribute__((aligned(2))) u32x2_any;
+        *(u32x2_any*)(po + (int64_t)v * VEC) = __builtin_bit_cast(u32x2, o.h[0]);
       } else {
 #pragma unroll
-        for (int w = 0; w < kBytes / 16; ++w) st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        for (int w = 0; w < kBytes / 16; ++w) {
+          if constexpr (ANY) st_stream_any<So>((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+          else st_stream((uint4*)(po + (int64_t)v * VEC) + w, o.u[w]);
+        }
       }
     }
   }
+  if (rem) po[tail] = ST<OutTag>::store(bwd_out<InTag, LOG>(rd, ry, s));
 }
 
+// Rows longer than the registers: the row sum in one read, the output in a
+// second, four 16-byte vectors of each operand per lane at a time.
 template <typename InTag, typename OutTag, bool LOG>
-__global__ __launch_bounds__(kBlock) void softmax_bwd_row_kernel(
+__global__ __launch_bounds__(kLong) void softmax_bwd_row_kernel(
     typename ST<OutTag>::storage* __restrict__ gi, const typename ST<InTag>::storage* __restrict__ dy,
     const typename ST<InTag>::storage* __restrict__ y, int64_t D) {
-  __shared__ float red[16];
+  typedef typename ST<InTag>::storage Si;
+  typedef typename ST<OutTag>::storage So;
+  constexpr int VEC = 16 / sizeof(Si);
+  __shared__ float red[kLong / 64];
+  union Vi {
+    uint4 u;
+    Si s[VEC];
+  };
   const int64_t row = blockIdx.x;
-  const typename ST<InTag>::storage* pd = dy + row * D;
-  const typename ST<InTag>::storage* py = y + row * D;
+  const Si* pd = dy + row * D;
+  const Si* py = y + row * D;
+  So* po = gi + row * D;
+  const int64_t nv = D / VEC, tail = nv * VEC + threadIdx.x;
+  auto load = [&](const Si* p, Vi* x, int64_t v0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)
+      x[u] = ld_stream_any<Si, Vi>(p + min(v0 + (int64_t)u * kLong, nv - 1) * VEC);
+  };
   float s = 0.f;
-  for (int64_t j = threadIdx.x; j < D; j += kBlock)
-    s += bwd_term<InTag, LOG>(ST<InTag>::load(pd[j]), ST<InTag>::load(py[j]));
-  s = block_sum_f(s, red);
-  typename ST<OutTag>::storage* po = gi + row * D;
-  for (int64_t j = threadIdx.x; j < D; j += kBlock)
-    po[j] = ST<OutTag>::store(bwd_out<InTag, LOG>(ST<InTag>::load(pd[j]), ST<InTag>::load(py[j]), s));
+  for (int64_t v0 = threadIdx.x; v0 < nv; v0 += kLong * kLongU) {
+    Vi xd[kLongU], xy[kLongU];
+    load(pd, xd, v0);
+    if constexpr (!LOG) load(py, xy, v0);
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u)
+      if (v0 + (int64_t)u * kLong < nv)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          s += bwd_term<InTag, LOG>(ST<InTag>::load(xd[u].s[e]),
+                                    LOG ? 0.f : ST<InTag>::load(xy[u].s[e]));
+  }
+  if (tail < D) s += bwd_term<InTag, LOG>(ST<InTag>::load(pd[tail]), ST<InTag>::load(py[tail]));
+  s = block_fsum<kLong>(s, red);
+  for (int64_t v0 = threadIdx.x; v0 < nv; v0 += kLong * kLongU) {
+    Vi xd[kLongU], xy[kLongU];
+    load(pd, xd, v0);
+    load(py, xy, v0);
+#pragma unroll
+    for (int u = 0; u < kLongU; ++u) {
+      const int64_t v = v0 + (int64_t)u * kLong;
+      if (v < nv) {
+        So o[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+          o[e] = ST<OutTag>::store(
+              bwd_out<InTag, LOG>(ST<InTag>::load(xd[u].s[e]), ST<InTag>::load(xy[u].s[e]), s));
+        __builtin_memcpy(po + v * VEC, o, sizeof(o));  // 8 or 16 bytes at element alignment
+      }
+    }
+  }
+  if (tail < D)
+    po[tail] = ST<OutTag>::store(
+        bwd_out<InTag, LOG>(ST<InTag>::load(pd[tail]), ST<InTag>::load(py[tail]), s));
 }
 
 template <typename InTag, typename OutTag, bool LOG>
@@ -420,15 +544,23 @@ mi_status_t launch_bwd_t(const mi_tensor_t* gi, const mi_tensor_t* dy, const mi_
     auto run_reg = [&](auto nth_c, auto vpt_c) -> mi_status_t {
       constexpr int NTH = decltype(nth_c)::value;
       constexpr int VPT = decltype(vpt_c)::value;
-      hipLaunchKernelGGL((softmax_bwd_reg_kernel<InTag, OutTag, NTH, VPT, LOG>),
-                         dim3((unsigned)outer), dim3(NTH), 0, stream, (So*)gi->data,
-                         (const Si*)dy->data, (const Si*)y->data, D);
+      const dim3 grid((unsigned)(NTH == 64 ? (outer + 3) / 4 : outer)), block(NTH, NTH == 64 ? 4 : 1);
+      if (aligned)
+        hipLaunchKernelGGL((softmax_bwd_reg_kernel<InTag, OutTag, NTH, VPT, LOG, false>), grid, block,
+                           0, stream, (So*)gi->data, (const Si*)dy->data, (const Si*)y->data, outer,
+                           D);
+      else
+        hipLaunchKernelGGL((softmax_bwd_reg_kernel<InTag, OutTag, NTH, VPT, LOG, true>), grid, block, 0,
+                           stream, (So*)gi->data, (const Si*)dy->data, (const Si*)y->data, outer, D);
       return check_launch("softmax_bwd_reg");
     };
     typedef std::integral_constant<int, 1> V1;
+    typedef std::integral_constant<int, 64> N64;
     typedef std::integral_constant<int, 1024> N1024;
     // two row operands in registers: up to 8 vectors of each per lane
-    if (aligned && nv <= 1024 * 8 && outer <= 0x7fffffff) {
+    if (nv <= 1024 * 8 && outer <= 0x7fffffff) {
+      if (nv <= 64) return run_reg(N64(), V1());
+      if (nv <= 128) return run_reg(N64(), std::integral_constant<int, 2>());
       if (nv <= 256) return run_reg(std::integral_constant<int, 256>(), V1());
       if (nv <= 512) return run_reg(std::integral_constant<int, 512>(), V1());
       if (nv <= 1024) return run_reg(N1024(), V1());
@@ -437,7 +569,7 @@ mi_status_t launch_bwd_t(const mi_tensor_t* gi, const mi_tensor_t* dy, const mi_
       return run_reg(N1024(), std::integral_constant<int, 8>());
     }
     hipLaunchKernelGGL((softmax_bwd_row_kernel<InTag, OutTag, LOG>), dim3((unsigned)outer),
-                       dim3(kBlock), 0, stream, (So*)gi->data, (const Si*)dy->data,
+                       dim3(kLong), 0, stream, (So*)gi->data, (const Si*)dy->data,
                        (const Si*)y->data, D);
     return check_launch("softmax_bwd_row");
   }
