@@ -382,3 +382,25 @@ def test_attention_few_queries_long_cache(dtype, B, H, Hk, Sq, Sk, D, form):
     _abi.flash_attention_fwd(out, lse, *dev, False, scale)
     assert_close(out, ref, "bf16", f"few queries {B},{H},{Hk},{Sq},{Sk},{D} {form}")
     assert (lse.cpu() - ref_lse).abs().max().item() < 2e-2 * max(1.0, ref_lse.abs().max().item())
+
+
+@pytest.mark.parametrize("B,H,Hk,S,D", [(1, 8, 8, 300, 128), (2, 8, 2, 260, 64), (4, 6, 3, 520, 128),
+                                        (3, 8, 8, 129, 64)])
+def test_causal_attention_head_groups(B, H, Hk, S, D):
+    """Causal query tiles of several heads interleaved (1 to 3 heads per XCD
+    with 2 to 5 query tiles each): every (head, tile) is computed once."""
+    q, k, v = rn((B, H, S, D), 91), rn((B, Hk, S, D), 92), rn((B, Hk, S, D), 93)
+    out = torch.full((B, H, S, D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    lse = torch.full((B, H, S), float("nan"), device="cuda")
+    _abi.flash_attention_fwd(out, lse, q.cuda(), k.cuda(), v.cuda(), True)
+    kk, vv = (t.repeat_interleave(H // Hk, 1).float().numpy() for t in (k, v))
+    ref, ref_lse = npr.attention64(q.float().numpy(), kk, vv, True, None)
+    mag, _ = npr.attention64(q.float().numpy(), kk, abs(vv), True, None)
+    # each weight is rounded to bf16 (8 significant bits: at most 2^-8 of it) and
+    # the output once more (2^-8 of it); a tenth more covers the fp32 scores, exponentials and sums.  The
+    # bf16 bar is too tight on rows of few keys, whose weights do not average
+    # (one of 307200 elements was 2.8e-3 off CPU ATen's own rounding)
+    bound = 1.1 * 2.0 ** -8 * (torch.from_numpy(mag) + torch.from_numpy(abs(ref))).double() + 1e-6
+    err = (out.cpu().double() - torch.from_numpy(ref).double()).abs()
+    assert bool((err <= bound).all()), (err / bound).max()
+    assert (lse.cpu().double() - torch.from_numpy(ref_lse).double()).abs().max().item() < 1e-3

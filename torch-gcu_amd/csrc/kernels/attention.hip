@@ -27,11 +27,14 @@
 //      through LDS; the V^T operand comes from V [key][d] by
 //      ds_read_b64_tr_b16, which hands each lane one d for 4 consecutive
 //      keys.
-// Key tiles above a wave's causal diagonal are skipped.  Blocks are ordered
-// head-major with the longest query tiles first, and renumbered so each of
-// the 8 XCDs (which receive workgroups round robin) walks a contiguous run of
-// heads: a head's K/V is then read into one XCD's L2 while its query tiles
-// run there.
+// Key tiles above a wave's causal diagonal are skipped.  Blocks are renumbered
+// so that each of the 8 XCDs (which receive workgroups round robin) walks a
+// contiguous run of heads: a head's K/V is then read into one XCD's L2 while its
+// query tiles run there.  With a causal mask the tiles of a group of heads are
+// interleaved longest first, the group as large as its K and V fit the L2: head
+// by head, each head's longest tile started late and the last ones ran alone.
+#include <algorithm>
+
 #include "attention_common.h"
 
 namespace mi {
@@ -81,11 +84,13 @@ __global__ __launch_bounds__(NT, 2) void flash_fwd_kernel(AttnArgs p) {
   __shared__ __align__(16) uint16_t vs0[C::TILE];
   __shared__ __align__(16) uint16_t vs1[C::TILE];
 
-  // block -> (b, h, query tile); head-major, longest query tile first
+  // block -> (b, h, query tile); a group of heads at a time, its longest query
+  // tiles first
   int bid = (int)blockIdx.x;
   if (p.xcd_remap) bid = (bid & 7) * (p.n_blocks >> 3) + (bid >> 3);
-  const int qt = p.q_tiles - 1 - bid % p.q_tiles;
-  const int bh = bid / p.q_tiles;
+  const int in_group = bid % (p.head_group * p.q_tiles);
+  const int qt = p.q_tiles - 1 - in_group / p.head_group;
+  const int bh = bid / (p.head_group * p.q_tiles) * p.head_group + in_group % p.head_group;
   const int64_t h = bh % p.H, b = bh / p.H;
   const int64_t hk = h * p.Hk / p.H;
   // the wave index read as wave-uniform: the loop bounds and tile bases
@@ -542,6 +547,18 @@ extern "C" mi_status_t mi_flash_attention_fwd(const mi_tensor_t* out, const mi_t
   MI_CHECK_ARG(nb <= 0x7fffffff, "attention: too many query tiles");
   a.n_blocks = (int)nb;
   a.xcd_remap = (nb % 8 == 0) ? 1 : 0;
+  a.head_group = 1;
+  if (a.causal && B * H % 8 == 0) {
+    // the heads of one XCD in equal groups of at most 8 MB of K and V (twice its
+    // L2; groups of 4 and 8 MB time the same where both divide the heads).  us,
+    // head by head and so: [4, 32 (8 k/v), 1500, 128] 136 -> 115, [8, 32, 2048,
+    // 128] 405 -> 383, [4, 32, 2048, 128] 219 -> 197, [1, 32, 3195, 128] 136 ->
+    // 117, [8, 32, 512, 128] 52 -> 46
+    const int64_t heads = B * H / 8, kv = Sk * D * 4;
+    const int64_t most = std::max<int64_t>(2, (8 << 20) / kv) * (H / Hk);
+    for (int64_t g = 1; g <= heads; ++g)
+      if (heads % g == 0 && g <= most) a.head_group = (int)g;
+  }
   hipStream_t s = (hipStream_t)stream;
   mi_status_t st;
   if (flash_decode(a, B, D, q->dtype == MI_F16, s, &st)) return st;

@@ -23,6 +23,7 @@ struct AttnArgs {
   float scale_log2;  // softmax scale * log2(e)
   int causal;
   int q_tiles;
+  int head_group;    // (b, h) pairs whose query tiles are interleaved, longest first
   int n_blocks;      // q_tiles * H * B
   int xcd_remap;     // n_blocks % 8 == 0: renumber blocks per XCD
 };
