@@ -140,3 +140,21 @@ def test_efficient_ops_on_gcu_tensors():
     want = torch.gcu.efficient.silu_mul(F.linear(x, w), F.linear(x, wu))
     assert got.shape == want.shape
     assert_equal_bits(got, want, "efficient.linear_silu_mul")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(65, 64, 64), (65, 1030, 128), (168, 4096, 512), (300, 1000, 1024),
+                                   (777, 520, 192), (1500, 2049, 256), (168, 512, 8192)])
+def test_fused_epilogues_on_every_tile_shape(dtype, M, N, K):
+    """linear_residual and linear_silu_mul below the large-tile sizes: the bits
+    of linear + add and of linear, linear, silu_mul, whichever kernels take them
+    (ragged tiles; the last shape is sliced along K and stays unfused)."""
+    gen = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=gen).to(dtype).to("gcu")
+    wg, wu = ((torch.randn(N, K, generator=gen) * 0.05).to(dtype).to("gcu") for _ in range(2))
+    r = torch.randn(M, N, generator=gen).to(dtype).to("gcu")
+    F = torch.nn.functional
+    ef = torch.gcu.efficient
+    assert torch.equal(ef.linear_residual(x, wg, r).cpu(), (r + F.linear(x, wg)).cpu())
+    assert torch.equal(ef.linear_silu_mul(x, wg, wu).cpu(),
+                       ef.silu_mul(F.linear(x, wg), F.linear(x, wu)).cpu())

@@ -1042,28 +1042,6 @@ mi_status_t launch_dl(const GemmArgs& q0, int64_t batch, hipStream_t s, const ch
   return check_launch(what);
 }
 
-// The large-tile kernel with a fused epilogue (EPI_RESID, EPI_SILU): 256 x 256
-// tiles over the output, or over 128 output columns (a gate and an up half)
-// for EPI_SILU.
-template <typename T, int EPI>
-mi_status_t launch_dl_epi(const GemmArgs& q0, hipStream_t s, const char* what) {
-  constexpr size_t lds = dl::LDS_BYTES;
-  static bool attr = [] {
-    (void)hipFuncSetAttribute((const void*)gemm_dl_kernel<T, false, false, false, false, EPI>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    return true;
-  }();
-  (void)attr;
-  GemmArgs q = q0;
-  const int64_t bn = EPI == EPI_SILU ? dl::BN / 2 : dl::BN;
-  q.tiles_m = (int)((q.M + dl::BM - 1) / dl::BM);
-  q.tiles_n = (int)((q.N + bn - 1) / bn);
-  hipLaunchKernelGGL((gemm_dl_kernel<T, false, false, false, false, EPI>),
-                     dim3((unsigned)(q.tiles_m * q.tiles_n)), dim3(dl::NT), lds, s, q, nullptr,
-                     (int64_t)0);
-  return check_launch(what);
-}
-
 // Row-major [K][N] B read in place by the large-tile kernel: enough tiles to
 // fill the CUs, K % 64 == 0, 16-byte aligned rows of both operands, N a
 // multiple of 8 (whole 16-byte column chunks) and 32-bit lane offsets.
@@ -1488,10 +1466,10 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
 // x [M, K] @ W^T with W [N, K] (a linear layer's weight) and a fused
 // epilogue: EPI_RESID adds `aux` (residual [M, N]) to the rounded product,
 // EPI_SILU multiplies silu(x Wg^T) by x Wu^T (W = Wg, aux = Wu), each product
-// rounded first, as the unfused ops do.  The large-tile kernel takes the whole
-// op when it applies (tiles enough to fill the CUs and its alignment and
-// 32-bit offset rules); otherwise the products go to workspace through the
-// regular matmul and the elementwise op follows, with the same results.
+// rounded first, as the unfused ops do.  One kernel takes the whole op where its
+// alignment and 32-bit offset rules hold and gemm_mid.hip's cost rule has it
+// faster; otherwise the products go to workspace through the regular matmul and
+// the elementwise op follows, with the same results.
 mi_status_t run_linear_epi(int epi, const mi_tensor_t* out, const mi_tensor_t* x,
                            const mi_tensor_t* w, const mi_tensor_t* aux, hipStream_t stream,
                            const char* what) {
@@ -1541,15 +1519,8 @@ mi_status_t run_linear_epi(int epi, const mi_tensor_t* out, const mi_tensor_t* x
     q.res = (const uint16_t*)aux->data;
     q.ldr = aux->strides[0];
   }
-  const int64_t bn = epi == EPI_SILU ? dl::BN / 2 : dl::BN;
-  fused = fused && ((M + dl::BM - 1) / dl::BM) * ((N + bn - 1) / bn) >= cu_count();
-  if (fused) {
-    if (dt == MI_BF16)
-      return epi == EPI_SILU ? launch_dl_epi<BF16, EPI_SILU>(q, stream, what)
-                             : launch_dl_epi<BF16, EPI_RESID>(q, stream, what);
-    return epi == EPI_SILU ? launch_dl_epi<F16, EPI_SILU>(q, stream, what)
-                           : launch_dl_epi<F16, EPI_RESID>(q, stream, what);
-  }
+  mi_status_t st;
+  if (fused && launch_gemm_fused(q, epi == EPI_SILU, dt == MI_F16, stream, what, &st)) return st;
   // unfused: the product(s) into workspace, then the elementwise op
   auto wt = [](const mi_tensor_t* t) {  // [K, N] view of a [N, K] weight
     mi_tensor_t v = *t;

@@ -37,6 +37,10 @@ mi_status_t launch_gemm_rows(const GemmArgs& q, bool f16, bool has_bias, hipStre
 bool gemm_mid_eligible(const GemmArgs& q);
 mi_status_t launch_gemm_mid(const GemmArgs& q, int64_t batch, bool f16, bool has_bias,
                             hipStream_t s, const char* what);
+// linear_residual / linear_silu_mul in one kernel (K a multiple of 64); returns
+// whether the call was taken, *st is its status then.
+bool launch_gemm_fused(const GemmArgs& q, bool silu, bool f16, hipStream_t s, const char* what,
+                       mi_status_t* st);
 // out = alpha * scale[n] * sum_s part[s] + beta * bias over S slices of raw
 // sums [M][ldp] (gemm.hip).
 mi_status_t launch_splitk_combine(const GemmArgs& q, bool f16, bool has_bias, const float* part,

@@ -80,23 +80,22 @@ constexpr int kSlices[] = {1, 2, 3, 4, 6, 8};
 
 struct Pick {
   int shape, slices;
+  float cost;
 };
 
-Pick pick_shape(const GemmArgs& q, int64_t batch) {
+// bn_div 2: a tile's columns are half gate and half up columns (EPI_SILU)
+Pick pick_shape(const GemmArgs& q, int64_t batch, bool split, int bn_div) {
   const int64_t steps = (q.K + 63) / 64, cus = cu_count();
-  // linear_residual and linear_silu_mul promise the unfused ops' bits: where
-  // their fused kernels run (256 x 256 or 256 x 128 tiles enough for the CUs)
-  // a product is summed in one piece
-  const bool split =
-      batch == 1 && ((q.M + 255) / 256) * ((q.N + 127) / 128) < cus;
-  const bool full = ((q.M + 255) / 256) * ((q.N + 255) / 256) * batch >= cus;
-  Pick best{0, 1};
-  float cost = 3e38f;
+  auto tiles_of = [&](int bm, int bn) {
+    return ((q.M + bm - 1) / bm) * ((q.N + bn / bn_div - 1) / (bn / bn_div)) * batch;
+  };
+  const bool full = tiles_of(256, 256) >= cus;
+  Pick best{0, 1, 3e38f};
   for (int i = 0; i < 5; ++i) {
     const Shape& c = kShapes[i];
-    const int64_t tiles = ((q.M + c.bm - 1) / c.bm) * ((q.N + c.bn - 1) / c.bn) * batch;
+    const int64_t tiles = tiles_of(c.bm, c.bn);
     for (int s : kSlices) {
-      if (s > 1 && (!split || steps < s || tiles * s > 4 * cus)) break;
+      if (s > 1 && (!split || batch > 1 || steps < s || tiles * s > 4 * cus)) break;
       const int64_t blocks = tiles * s, rounds = (blocks + cus - 1) / cus;
       const float load = std::min(1.f, (float)blocks / (float)cus);
       float t = c.fixed + (float)(rounds * ((steps + s - 1) / s)) * (c.lo + (c.hi - c.lo) * load) +
@@ -106,10 +105,7 @@ Pick pick_shape(const GemmArgs& q, int64_t batch) {
       // the sustained clock they lose about that much (M6000 N11008 K4096, 1 %
       // apart by this rule: 481 us on 256 x 256 tiles, 506 on 256 x 128)
       if (i > 0 && full) t *= 1.05f;
-      if (t < cost) {
-        cost = t;
-        best = Pick{i, s};
-      }
+      if (t < best.cost) best = Pick{i, s, t};
     }
   }
   return best;
@@ -126,6 +122,35 @@ mi_status_t run(const GemmArgs& q, Pick c, int64_t batch, hipStream_t s, const c
   }
 }
 
+template <typename T, int EPI, class C>
+mi_status_t launch_epi(const GemmArgs& q0, hipStream_t s, const char* what) {
+  static bool attr = [] {
+    (void)hipFuncSetAttribute((const void*)gemm_dl_kernel<T, false, false, false, false, EPI, C>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES);
+    return true;
+  }();
+  (void)attr;
+  GemmArgs q = q0;
+  constexpr int BN = EPI == EPI_SILU ? C::BN / 2 : C::BN;
+  q.tiles_m = (int)((q.M + C::BM - 1) / C::BM);
+  q.tiles_n = (int)((q.N + BN - 1) / BN);
+  hipLaunchKernelGGL((gemm_dl_kernel<T, false, false, false, false, EPI, C>),
+                     dim3((unsigned)(q.tiles_m * q.tiles_n)), dim3(C::NT), C::LDS_BYTES, s, q, nullptr,
+                     (int64_t)0);
+  return check_launch(what);
+}
+
+template <typename T, int EPI>
+mi_status_t run_epi(const GemmArgs& q, int shape, hipStream_t s, const char* what) {
+  switch (shape) {
+    case 0: return launch_epi<T, EPI, C256>(q, s, what);
+    case 1: return launch_epi<T, EPI, C256x128>(q, s, what);
+    case 2: return launch_epi<T, EPI, C128>(q, s, what);
+    case 3: return launch_epi<T, EPI, C128x64>(q, s, what);
+    default: return launch_epi<T, EPI, C64>(q, s, what);
+  }
+}
+
 }  // namespace
 
 bool gemm_mid_eligible(const GemmArgs& q) {
@@ -138,10 +163,29 @@ bool gemm_mid_eligible(const GemmArgs& q) {
 
 mi_status_t launch_gemm_mid(const GemmArgs& q, int64_t batch, bool f16, bool has_bias, hipStream_t s,
                             const char* what) {
-  const Pick c = pick_shape(q, batch);
+  const Pick c = pick_shape(q, batch, true, 1);
   if (f16)
     return has_bias ? run<F16, true>(q, c, batch, s, what) : run<F16, false>(q, c, batch, s, what);
   return has_bias ? run<BF16, true>(q, c, batch, s, what) : run<BF16, false>(q, c, batch, s, what);
+}
+
+// A fused epilogue (residual add, or SiLU-mul of two products) on the tile
+// shape of least cost.  Its bits are the unfused ops' only if those sum K in one
+// piece, so a product that launch_gemm_mid would slice is left to them (its
+// slices are also what makes it fast), and so is one whose products and
+// elementwise pass cost less.  us, unfused and fused: gate / up of 168 tokens
+// (N11008 K4096) 91 -> 62; on the 256 x 256 tiles alone before, 1496 tokens
+// (N5504 K2048, 258 tiles) 94 -> 76.
+bool launch_gemm_fused(const GemmArgs& q, bool silu, bool f16, hipStream_t s, const char* what,
+                       mi_status_t* st) {
+  const Pick plain = pick_shape(q, 1, true, 1);
+  if (plain.slices > 1) return false;
+  const Pick c = pick_shape(q, 1, false, silu ? 2 : 1);
+  const float pass = 3.f + (float)q.M * (float)q.N * (6.f / 5.8e6f);
+  if (c.cost > (silu ? 2.f : 1.f) * plain.cost + pass) return false;
+  if (silu) *st = f16 ? run_epi<F16, EPI_SILU>(q, c.shape, s, what) : run_epi<BF16, EPI_SILU>(q, c.shape, s, what);
+  else *st = f16 ? run_epi<F16, EPI_RESID>(q, c.shape, s, what) : run_epi<BF16, EPI_RESID>(q, c.shape, s, what);
+  return true;
 }
 
 }  // namespace mi
