@@ -785,3 +785,19 @@ def test_row_reductions_of_short_rows_at_any_offset(dtype):
         s = torch.empty(rows, dtype=sd, device="cuda")
         _abi.sum_(s, xd, [-1])
         assert_exact(s, x.sum(-1, dtype=sd), f"sum {rows}x{width}")
+
+
+@pytest.mark.parametrize("dtype", [torch.uint8, torch.bfloat16, torch.float32, torch.int64])
+@pytest.mark.parametrize("rows,width,pad_in,pad_out", [(7, 64, 1, 0), (300, 65, 0, 3), (33, 1001, 3, 5),
+                                                       (2, 100003, 1, 1), (5000, 67, 0, 1)])
+def test_copy_of_contiguous_rows(dtype, rows, width, pad_in, pad_out):
+    """Row-contiguous copies between different row strides, at odd lengths and
+    offsets; bytes outside the rows stay."""
+    gen = torch.Generator().manual_seed(rows)
+    src = torch.randint(0, 200, (3, rows, width + pad_in), generator=gen).to(dtype)
+    dst = torch.full((3, rows, width + pad_out), 77).to(dtype)
+    ddst = dst.cuda()
+    sv, dv = src[:, :, pad_in:], ddst[:, :, pad_out:]
+    _abi.copy_(dv, src.cuda()[:, :, pad_in:])
+    dst[:, :, pad_out:] = sv
+    assert torch.equal(ddst.cpu(), dst)

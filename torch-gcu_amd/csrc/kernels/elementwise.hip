@@ -326,6 +326,34 @@ __global__ __launch_bounds__(kBlock) void copy_raw_kernel(T* out, const T* src,
   }
 }
 
+// Rows that are contiguous in both operands (a padded or sliced matrix, rows of
+// any length and offset): 16-byte accesses at element alignment, four in flight
+// per lane; a row's last piece is moved back to end with the row, where two
+// lanes then write the same bytes.  Element by element such copies ran at 1.4
+// TB/s (bf16 [3840, 3443] into rows of 3448: 37 us).
+__global__ __launch_bounds__(kBlock) void copy_rows_kernel(char* out, const char* src,
+                                                           OffsetCalc<2> oc, int esz, int64_t len,
+                                                           uint32_t pieces, int64_t total) {
+  constexpr int U = 4;
+  const int64_t i0 = (int64_t)blockIdx.x * (kBlock * U) + threadIdx.x;
+  typedef u32x4_t __attribute__((aligned(1))) any_t;
+  u32x4_t v[U];
+  char* dst[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t i = min(i0 + u * kBlock, total - 1);
+    const int64_t row = total <= 0xffffffffLL ? (int64_t)((uint32_t)i / pieces) : i / pieces;
+    const int64_t at = min((i - row * pieces) * 16, len - 16);
+    int64_t off[2];
+    oc.get(row, off);
+    dst[u] = out + off[0] * esz + at;
+    v[u] = __builtin_nontemporal_load((const any_t*)(src + off[1] * esz + at));
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (i0 + u * kBlock < total) *(any_t*)dst[u] = v[u];
+}
+
 // Contiguous float <-> half/bfloat16 conversion, 8 elements per thread.
 template <typename SrcTag, typename DstTag>
 __global__ __launch_bounds__(kBlock) void convert_contig_kernel(
@@ -773,6 +801,17 @@ mi_status_t mi_copy(const mi_tensor_t* out, const mi_tensor_t* src, mi_stream_t 
       }
     }
     OffsetCalc<2> oc = make_offset_calc<2>(it);
+    const int64_t len = it.sizes[nd - 1] * esz;
+    if (nd >= 2 && it.strides[0][nd - 1] == 1 && it.strides[1][nd - 1] == 1 && len >= 64 &&
+        len <= 0xffffffffLL) {
+      oc.ndim = nd - 1;  // the rows
+      const int64_t pieces = (len + 15) / 16, total = it.numel / it.sizes[nd - 1] * pieces;
+      if (total <= (int64_t)kBlock * 4 * 0x7fffffff) {
+        hipLaunchKernelGGL(copy_rows_kernel, dim3(ceil_div_u(total, kBlock * 4)), dim3(kBlock), 0,
+                           stream, it.data[0], it.data[1], oc, esz, len, (uint32_t)pieces, total);
+        return check_launch("copy_rows");
+      }
+    }
     const unsigned g = grid_for(it.numel);
     switch (esz) {
       case 1: hipLaunchKernelGGL(copy_raw_kernel<uint8_t>, dim3(g), dim3(kBlock), 0, stream, (uint8_t*)it.data[0], (const uint8_t*)it.data[1], oc, it.numel); break;
