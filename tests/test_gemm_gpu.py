@@ -617,3 +617,28 @@ def test_f32_bmm_layouts():
     for bb in (b.cuda(), b.transpose(1, 2).contiguous().cuda().transpose(1, 2)):
         _abi.bmm(out, a.cuda(), bb)
         assert_close(out, torch.bmm(a.double(), b.double()).float(), "fp32", "f32 bmm")
+
+
+@pytest.mark.parametrize("M,N,K,dtype,bias", [
+    (1, 17, 1, torch.bfloat16, None), (8, 100, 127, torch.float16, "f32"),
+    (16, 4096, 2048, torch.bfloat16, "bf16"), (15, 1920, 1083, torch.float16, None),
+    (17, 8200, 129, torch.bfloat16, None), (48, 63, 384, torch.bfloat16, "f32"),
+    (33, 70, 16511, torch.bfloat16, None), (64, 1000, 8320, torch.float16, "f32"),
+    (600, 1000, 1024, torch.bfloat16, None), (3000, 2100, 128, torch.bfloat16, "f32"),
+])
+def test_int8_linear_any_k(M, N, K, dtype, bias):
+    """The few-row kernel with an int8 weight (any K, a unit of 128 and its
+    remainder, weight rows and x at odd offsets, K slices) and, above 512 rows,
+    sliced and whole 256 x 256 tiles."""
+    x = rn((M, K), 90, dtype, 1.0)
+    w = torch.randint(-127, 128, (N, K), generator=g(91), dtype=torch.int8)
+    sc = torch.rand(N, generator=g(92)) * 0.009 + 0.001
+    b = None if bias is None else (torch.randn(N, generator=g(93)) if bias == "f32" else rn((N,), 93, dtype, 1.0))
+    ref = aten.int8_linear(x, w, sc, b)
+    buf = torch.empty(N * K + 1, dtype=torch.int8, device="cuda")
+    buf[1:].copy_(w.reshape(-1))
+    for wd in (w.cuda(), buf[1:].view(N, K)):
+        out = torch.full((M, N + 1), 7.0, dtype=dtype, device="cuda")
+        _abi.int8_linear(out[:, :N], x.cuda(), wd, sc.cuda(), None if b is None else b.cuda())
+        assert_close(out[:, :N], ref, "bf16", f"int8 {M}x{N}x{K}")
+        assert bool((out[:, N] == 7.0).all())

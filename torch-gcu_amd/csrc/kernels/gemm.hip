@@ -557,21 +557,6 @@ mi_status_t launch_mid(const GemmArgs& q0, hipStream_t s, const char* what) {
   return check_launch(what);
 }
 
-// ---- int8 weight-only linear for few rows (M <= 64): HBM-bound on W -------------------
-//
-// A 512-lane block owns 32 output columns (two 16-row tiles of W [N, K]);
-// its 8 waves split K into interleaved 128-wide chunks, so per step the block
-// reads 1 KiB contiguous bytes of each of its W rows and every 128-byte line
-// is read whole by one wave.  In a chunk, lane (r = l % 16, g = l / 16)
-// streams W[n0 + 16 t + r][128 c + 32 g .. + 32] with two non-temporal
-// 16-byte loads per tile t, widens the 32 int8 to bf16 (exact) and feeds
-// v_mfma_f32_16x16x32 with the matching 32 k of each x row (x is [M, K] and
-// stays in cache).  The k order inside a chunk is the same for both
-// operands, so the sum is the plain dot product.  The 8 waves' partial
-// 16 x 16 tiles are added in a fixed order through LDS; the epilogue applies
-// the per-column scale and bias and rounds once.
-typedef int int4v_t __attribute__((ext_vector_type(4)));
-
 template <typename T>
 struct Mfma16;
 template <>
@@ -580,15 +565,6 @@ struct Mfma16<BF16> {
   static __device__ __forceinline__ f32x4_t mma(vec a, vec b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ vec widen(int4v_t w, int half) {
-    vec v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int byte = 8 * half + e;
-      v[e] = (__bf16)(float)(int8_t)(w[byte >> 2] >> (8 * (byte & 3)));
-    }
-    return v;
-  }
 };
 template <>
 struct Mfma16<F16> {
@@ -596,139 +572,12 @@ struct Mfma16<F16> {
   static __device__ __forceinline__ f32x4_t mma(vec a, vec b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
-  static __device__ __forceinline__ vec widen(int4v_t w, int half) {
-    vec v;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int byte = 8 * half + e;
-      v[e] = (_Float16)(float)(int8_t)(w[byte >> 2] >> (8 * (byte & 3)));
-    }
-    return v;
-  }
 };
-
-constexpr int kSkN = 2;    // 16-row n-tiles per block (32 W rows)
-constexpr int kSkW = 8;    // waves per block, splitting K
-
-template <typename T, int MT, bool HAS_BIAS>
-__global__ __launch_bounds__(64 * kSkW, MT == 1 ? 4 : 1) void int8_skinny_kernel(GemmArgs p) {
-  typedef typename Mfma16<T>::vec vec;
-  __shared__ float red[kSkW][kSkN][16][17];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 15, g = lane >> 4;
-  const int64_t n0 = (int64_t)blockIdx.x * 16 * kSkN;
-  // lane (r, g) owns bytes [32 g, 32 g + 32) of each 128-byte chunk of the W
-  // rows n0 + 16 t + r, so one wave reads whole 128-byte lines
-  const int8_t* wrow[kSkN];
-#pragma unroll
-  for (int t = 0; t < kSkN; ++t)
-    wrow[t] = (const int8_t*)p.b + min<int64_t>(n0 + 16 * t + r, p.N - 1) * p.ldb + 32 * g;
-  const uint16_t* xrow[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-    xrow[mt] = p.a + min<int64_t>(mt * 16 + r, p.M - 1) * p.lda + 32 * g;
-  f32x4_t acc[MT][kSkN];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int t = 0; t < kSkN; ++t) acc[mt][t] = f32x4_t{};
-  // one 128-wide chunk of W (kSkN tiles) and x in registers, double-buffered:
-  // the loads of chunk c + kSkW are in flight while chunk c is widened and
-  // multiplied
-  struct Chunk {
-    int4v_t w[kSkN][2];
-    vec x[MT][4];
-  };
-  auto load = [&](Chunk& ch, int c) __attribute__((always_inline)) {
-#pragma unroll
-    for (int t = 0; t < kSkN; ++t) {
-      const int8_t* wp = wrow[t] + 128 * c;
-      ch.w[t][0] = __builtin_bit_cast(int4v_t, ld_stream((const uint4*)wp));
-      ch.w[t][1] = __builtin_bit_cast(int4v_t, ld_stream((const uint4*)(wp + 16)));
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int h = 0; h < 4; ++h) ch.x[mt][h] = *(const vec*)(xrow[mt] + 128 * c + 8 * h);
-  };
-  // consecutive MFMAs go to different accumulators (n-tiles inner)
-  auto compute = [&](const Chunk& ch) __attribute__((always_inline)) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-      for (int t = 0; t < kSkN; ++t) {
-        // the empty asm pins the start of the byte unpacking here, so the
-        // compiler cannot unpack every loaded W byte into its own register
-        // right after the loads
-        int4v_t wd = ch.w[t][h >> 1];
-        asm volatile("" : "+v"(wd));
-        const vec wk = Mfma16<T>::widen(wd, h & 1);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt][t] = Mfma16<T>::mma(ch.x[mt][h], wk, acc[mt][t]);
-      }
-  };
-  const int KC = (int)(p.K / 128);  // chunks; wave w takes chunks w, w + kSkW, ...
-  // two named buffers (a runtime-indexed pair would live in scratch memory)
-  Chunk b0, b1;
-  if (wave < KC) load(b0, wave);
-  for (int c = wave; c < KC; c += 2 * kSkW) {
-    if (c + kSkW < KC) load(b1, c + kSkW);
-    compute(b0);
-    if (c + kSkW < KC) {
-      if (c + 2 * kSkW < KC) load(b0, c + 2 * kSkW);
-      compute(b1);
-    }
-  }
-  // D[m = 4 (l / 16) + i][n = l % 16] of each 16 x 16 (m-tile, n-tile); the
-  // m-tiles are reduced one at a time through LDS
-  const int tn = threadIdx.x & 15, tm = (threadIdx.x >> 4) & 15, tt = threadIdx.x >> 8;
-  const bool bias_f32 = p.bias_dtype == MI_F32;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    if (mt > 0) __syncthreads();
-#pragma unroll
-    for (int t = 0; t < kSkN; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][t][4 * g + i][r] = acc[mt][t][i];
-    __syncthreads();
-    const int64_t m = mt * 16 + tm;
-    if (m >= p.M) continue;
-    // 512 lanes: lane -> (n-tile tt (+2, ...), row m, column n)
-#pragma unroll
-    for (int t = tt; t < kSkN; t += 2) {
-      const int64_t n = n0 + 16 * t + tn;
-      if (n >= p.N) continue;
-      float sum = red[0][t][tm][tn];
-#pragma unroll
-      for (int w = 1; w < kSkW; ++w) sum += red[w][t][tm][tn];
-      float v = p.alpha * p.scale[n] * sum;
-      if (HAS_BIAS) {
-        const int64_t bo = m * p.bias_sm + n * p.bias_sn;
-        v += p.beta * (bias_f32 ? ((const float*)p.bias)[bo]
-                                : MfmaOp<T>::load(((const uint16_t*)p.bias)[bo]));
-      }
-      p.c[m * p.ldc + n] = MfmaOp<T>::store(v);
-    }
-  }
-}
-
-template <typename T, bool HB>
-mi_status_t launch_skinny(const GemmArgs& q, hipStream_t s) {
-  const dim3 grid(ceil_div_u(q.N, 16 * kSkN)), block(64 * kSkW);
-  const int mt = (int)((q.M + 15) / 16);
-  switch (mt) {
-    case 1: hipLaunchKernelGGL((int8_skinny_kernel<T, 1, HB>), grid, block, 0, s, q); break;
-    case 2: hipLaunchKernelGGL((int8_skinny_kernel<T, 2, HB>), grid, block, 0, s, q); break;
-    case 3: hipLaunchKernelGGL((int8_skinny_kernel<T, 3, HB>), grid, block, 0, s, q); break;
-    default: hipLaunchKernelGGL((int8_skinny_kernel<T, 4, HB>), grid, block, 0, s, q); break;
-  }
-  return check_launch("int8_linear skinny");
-}
 
 // ---- int8 weight-only linear for few rows, weight staged through LDS ------------------
 //
-// The contraction of int8_skinny_kernel for K % 1024 == 0 and 16-byte aligned
-// W rows.  A 512-lane block owns R consecutive W rows, R = N / CUs rounded up
+// For M <= 64, K % 1024 == 0, 16-byte aligned W rows and enough of them
+// (gemm_rows.hip takes the rest): bound by the HBM stream of W.  A 512-lane block owns R consecutive W rows, R = N / CUs rounded up
 // (43 for N = 11008 on 256 CUs) and at most 48, so every CU streams the same
 // share of W once (with 32-row blocks, 344 blocks on 256 CUs left 88 CUs
 // streaming twice the bytes of the others).  K is walked in 1 KiB slabs of
@@ -1154,14 +1003,14 @@ mi_status_t launch_splitk(const GemmArgs& q0, int S, hipStream_t s, const char* 
 
 template <typename T, bool I8, bool HB>
 mi_status_t launch_mfma(const GemmArgs& q, int64_t batch, hipStream_t s, const char* what) {
-  // int8 W and 64 < M <= 512 (config 4's M = 256): split-K over 256 x 256
-  // tiles when they are too few to fill the CUs (M = 256: 43 tiles x 5 K
-  // slices, 43.6 us against 49.9 us for 128-row tiles over the whole K; M =
-  // 96 .. 512 all faster), else 128-row tiles sized to the CUs
-  if (I8 && batch == 1 && q.M > 64 && q.M <= 4 * mid::BM && dl_eligible(q, true)) {
+  // int8 W and 64 < M: split-K over 256 x 256 tiles when they are too few to fill
+  // the CUs (M = 256: 43 tiles x 5 K slices, 43.6 us against 49.9 us for 128-row
+  // tiles over the whole K; M = 96 .. 512 all faster; M2862 N2240 K4032, 108
+  // tiles x 2: 75 us against 107), else 128-row tiles sized to the CUs
+  if (I8 && batch == 1 && q.M > 64 && dl_eligible(q, true)) {
     const int S = splitk_slices(q);
     if (S > 1) return launch_splitk<T, HB, true>(q, S, s, what);
-    return launch_mid<T, HB>(q, s, what);
+    if (q.M <= 4 * mid::BM) return launch_mid<T, HB>(q, s, what);
   }
   if constexpr (!I8) {
     // tile shape and K slices by gemm_mid.hip's cost rule
@@ -1172,9 +1021,10 @@ mi_status_t launch_mfma(const GemmArgs& q, int64_t batch, hipStream_t s, const c
   } else {
     const int64_t cus = cu_count();
     const int64_t big = ((q.M + 255) / 256) * ((q.N + 255) / 256) * batch;
-    if (big >= cus && dl_eligible(q, true)) return launch_dl<T, HB, true>(q, batch, s, what);
+    // (too many tiles to slice: from half the CUs on, M3000 N4096 K4096 on 192
+    // tiles 102 us against 162 on 128 x 64 ones)
+    if (big >= cus / 2 && dl_eligible(q, true)) return launch_dl<T, HB, true>(q, batch, s, what);
     if (big >= cus) return Cfg<T, 256, 256, 2, 4, true, HB>::launch(q, batch, s, what);
-    if (q.M <= 32) return Cfg<T, 32, 64, 1, 2, true, HB>::launch(q, batch, s, what);
     // 128 x 64 tiles: twice the blocks of 128 x 128, so CUs hold two and overlap
     // one's loads with the other's MFMAs (about 15 % faster at M = 256)
     return Cfg<T, 128, 64, 2, 2, true, HB>::launch(q, batch, s, what);
@@ -1348,8 +1198,15 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
   // or B as row-major [K, N] rows read in place by the large-tile kernel
   Workspace wa, wb, wc;
   Mat Bt = transposed(B);
-  // few rows: the weight stream kernel, operands read as they are
-  if (!int8 && batch == 1 && M <= kRowsMax && (A.s1 == 1 || K == 1) && (Bt.s1 == 1 || K == 1) &&
+  // few rows: the weight stream kernels, operands read as they are.  An int8
+  // weight of whole 1 KiB slabs keeps int8_stream_kernel where its N / CUs rows
+  // per block are worth its 48-row slabs (M24 N11008 K4096 14.1 us against 16.4;
+  // M8 N4096 K4096 8.1 against 6.7, M64 N4096 K8192 39 against 19)
+  const bool stream8 = int8 && M <= 64 && K % kStSlab == 0 && N >= 32 * cu_count() && A.s1 == 1 &&
+                       (A.s0 % 8 == 0 || M == 1) && Bt.s1 == 1 && Bt.s0 % 16 == 0 &&
+                       ((((uintptr_t)A.data) | ((uintptr_t)B.data)) & 15) == 0 &&
+                       (C.s1 == 1 || N == 1);
+  if (!stream8 && batch == 1 && M <= kRowsMax && (A.s1 == 1 || K == 1) && (Bt.s1 == 1 || K == 1) &&
       (C.s1 == 1 || N == 1)) {
     GemmArgs q{};
     q.a = (const uint16_t*)A.data;
@@ -1365,6 +1222,7 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
     q.lda = A.s0;
     q.ldb = Bt.s0;
     q.ldc = C.s0;
+    q.scale = int8 ? (const float*)scale->data : nullptr;
     q.alpha = (float)alpha;
     q.beta = (float)beta;
     if (gemm_rows_eligible(q))
@@ -1431,25 +1289,12 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
     }
     return MI_OK;
   }
-  // int8 weight with few rows of x: the weight stream dominates
-  const bool skinny = int8 && batch == 1 && M <= 64 && K % 128 == 0 && (q.lda % 8) == 0 &&
-                      (q.ldb % 16) == 0 && ((((uintptr_t)q.a) | ((uintptr_t)q.b)) & 15) == 0 &&
-                      (N == 1 || Cw.s1 == 1);
-  // K in whole 1 KiB slabs: the LDS-staged weight stream; else the register one
-  const bool stream_ok = skinny && K % kStSlab == 0;
-  if (stream_ok) {
+  if (stream8) {
     mi_status_t st;
     if (A.dtype == MI_BF16)
       st = has_bias ? launch_stream<BF16, true>(q, stream) : launch_stream<BF16, false>(q, stream);
     else
       st = has_bias ? launch_stream<F16, true>(q, stream) : launch_stream<F16, false>(q, stream);
-    MI_RETURN_IF(st);
-  } else if (skinny) {
-    mi_status_t st;
-    if (A.dtype == MI_BF16)
-      st = has_bias ? launch_skinny<BF16, true>(q, stream) : launch_skinny<BF16, false>(q, stream);
-    else
-      st = has_bias ? launch_skinny<F16, true>(q, stream) : launch_skinny<F16, false>(q, stream);
     MI_RETURN_IF(st);
   } else if (A.dtype == MI_BF16) {
     MI_RETURN_IF(dispatch_mfma<BF16>(q, int8, has_bias, batch, stream, what));

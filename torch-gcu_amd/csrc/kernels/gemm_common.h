@@ -26,7 +26,8 @@ struct GemmArgs {
 };
 
 // Few-row products (gemm_rows.hip): out = alpha * a b^T + beta * bias with
-// M <= kRowsMax, one batch, K-contiguous 16-bit operands of any alignment.
+// M <= kRowsMax, one batch, K-contiguous operands of any alignment; b 16-bit, or
+// int8 when q.scale is set.
 constexpr int64_t kRowsMax = 64;
 bool gemm_rows_eligible(const GemmArgs& q);
 mi_status_t launch_gemm_rows(const GemmArgs& q, bool f16, bool has_bias, hipStream_t s,

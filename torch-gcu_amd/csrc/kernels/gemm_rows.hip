@@ -1,5 +1,6 @@
-// 16-bit matrix products with few rows: out[m][n] = alpha * sum_k a[m][k] b[n][k]
-// + beta * bias with M <= 64, the linear layers of a decode step.
+// Matrix products with few rows: out[m][n] = alpha * sum_k a[m][k] b[n][k]
+// + beta * bias with M <= 64, 16-bit a and a 16-bit or int8 b: the linear layers
+// of a decode step.
 //
 // What bounds it: the weight b [N][K] is streamed once from HBM and each of
 // its elements meets at most 64 rows, so the matrix cores idle and the time is
@@ -22,7 +23,7 @@
 //
 // Addresses need only the element's alignment (a global dwordx4 load may start
 // at any 2-byte address), so odd K, row strides and bases run here as they
-// are; the last K % 64 elements are read one by one by one wave.
+// are; the last K % 64 (int8: 128) elements are read one by one by one wave.
 #include <algorithm>
 
 #include "gemm_common.h"
@@ -37,13 +38,42 @@ __device__ __forceinline__ int swz(int r, int c) {
   return c ^ (r & 3) ^ (((r >> 2) & 1) * 5) ^ ((r >> 1) & 4);
 }
 
-template <typename T, int MT, int RT, int NW, bool HAS_BIAS, bool SPLIT>
+// out[m][n .. n + 3] = alpha * s (* scale[n]) + beta * bias, rounded once
+template <typename T, bool HAS_BIAS, bool I8>
+__device__ __forceinline__ void rows_store(const GemmArgs& p, int64_t m, int64_t n, f32x4_t s) {
+  f32x4_t bb = {}, sc = {1.f, 1.f, 1.f, 1.f};
+  if constexpr (I8) sc = load_col4_t<T>(p.scale, MI_F32, n, 1, p.N, 0);
+  if constexpr (HAS_BIAS)
+    bb = load_col4_t<T>(p.bias, p.bias_dtype, n, p.bias_sn, p.N, m * p.bias_sm);
+  u16x4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x = p.alpha * s[e];
+    if constexpr (I8) x *= sc[e];
+    if constexpr (HAS_BIAS) x += p.beta * bb[e];
+    v[e] = MfmaOp<T>::store(x);
+  }
+  uint16_t* dst = p.c + m * p.ldc + n;
+  if (n + 3 < p.N && (((uintptr_t)dst) & 7) == 0) {
+    *(u16x4_t*)dst = v;
+  } else {
+    for (int e = 0; e < 4 && n + e < p.N; ++e) dst[e] = v[e];
+  }
+}
+
+// I8: b is an int8 weight with fp32 scale per row (the int8 linear), its unit
+// 128 deep; a's 16 rows of a unit are then two tiles of 64.
+template <typename T, int MT, int RT, int NW, bool HAS_BIAS, bool SPLIT, bool I8>
 __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* part, int64_t ldp) {
   typedef typename MfmaOp<T>::vec vec;
   typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-  typedef u16x8 __attribute__((aligned(2))) u16x8_u;
-  constexpr int NT = RT + MT;          // 16-row operand tiles: RT of b, then MT of a
-  constexpr int TILE = 16 * 64;        // elements of one tile of a 64-deep unit
+  typedef u16x8 __attribute__((aligned(1))) u16x8_u1;
+  typedef u16x8 __attribute__((aligned(2))) u16x8_u2;
+  typedef typename std::conditional<I8, u16x8_u1, u16x8_u2>::type u16x8_u;
+  constexpr int XS = I8 ? 2 : 1, KU = 64 * XS;  // a tiles per 16 rows, k per unit
+  constexpr int BE = I8 ? 1 : 2;                // bytes per b element
+  constexpr int NT = RT + MT * XS;     // tiles of 16 rows x 128 bytes: RT of b, then a's
+  constexpr int TILE = 16 * 64;        // 16-bit elements of one tile
   constexpr int NTL = RT * MT;
   constexpr size_t kStage = (size_t)NW * NT * TILE * 2, kRed = (size_t)NW * NTL * 64 * 16;
   __shared__ __align__(16) char smem[kStage > kRed ? kStage : kRed];
@@ -54,19 +84,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
   // each 128-byte unit.  Per-lane byte offsets from a block-uniform base (the
   // host checked that they fit 32 bits); rows past the end re-read the last
   // one and feed outputs that are never stored
-  const char* base[2] = {(const char*)((const uint16_t*)p.b + n0 * p.ldb), (const char*)p.a};
+  const char* base[2] = {(const char*)p.b + n0 * p.ldb * BE, (const char*)p.a};
   uint32_t off[NT][2];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int row = 8 * h + (lane >> 3);
-      const int64_t gr = t < RT ? (min<int64_t>(n0 + 16 * t + row, p.N - 1) - n0) * p.ldb
-                                : min<int64_t>(16 * (t - RT) + row, p.M - 1) * p.lda;
-      off[t][h] = (uint32_t)(gr * 2 + 16 * (lane & 7));
+      const int mt = (t - RT) / XS, sub = (t - RT) % XS;
+      const int64_t at = t < RT
+                             ? (min<int64_t>(n0 + 16 * t + row, p.N - 1) - n0) * p.ldb * BE
+                             : min<int64_t>(16 * mt + row, p.M - 1) * p.lda * 2 + 128 * sub;
+      off[t][h] = (uint32_t)(at + 16 * (lane & 7));
     }
   uint16_t* tile = (uint16_t*)smem + wave * (NT * TILE);
-  int wo[2], ro[2];
+  int wo[2], ro[2], ro8[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)  // int8 k 32 s + 8 (l / 16) .. + 7
+    ro8[s] = (lane & 15) * 64 + 8 * swz(lane & 15, 2 * s + (lane >> 5)) + 4 * ((lane >> 4) & 1);
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int row = 8 * h + (lane >> 3);
@@ -84,7 +119,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
     else
       return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   };
-  // one 64-deep unit: the loaded rows through the wave's own LDS tiles into
+  // one unit: the loaded rows through the wave's own LDS tiles into
   // MFMA fragments (LDS operations of a wave stay in order)
   struct Unit {
     u16x8 v[NT][2];
@@ -98,14 +133,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      vec f[NT];
+    for (int s = 0; s < KU / 32; ++s) {
+      vec fw[RT], fx[MT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) f[t] = *(const vec*)(tile + t * TILE + ro[s]);
+      for (int i = 0; i < RT; ++i) {
+        if constexpr (I8) fw[i] = widen8<T>(*(const u32x2_t*)(tile + i * TILE + ro8[s]));
+        else fw[i] = *(const vec*)(tile + i * TILE + ro[s]);
+      }
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+        fx[j] = *(const vec*)(tile + (RT + XS * j + s / 2) * TILE + ro[s & 1]);
 #pragma unroll
       for (int i = 0; i < RT; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j) acc[i][j] = mma(f[i], f[RT + j], acc[i][j]);
+        for (int j = 0; j < MT; ++j) acc[i][j] = mma(fw[i], fx[j], acc[i][j]);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -113,8 +154,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
   };
 
   // whole units k_first .. KS - 1 of this block's K slice
-  int KS = (int)(p.K / 64), k_first = 0;
-  const bool has_tail = KS * (int64_t)64 < p.K && (!SPLIT || blockIdx.y + 1 == gridDim.y);
+  int KS = (int)(p.K / KU), k_first = 0;
+  const bool has_tail = KS * (int64_t)KU < p.K && (!SPLIT || blockIdx.y + 1 == gridDim.y);
   if constexpr (SPLIT) {
     const int per = KS / (int)gridDim.y, rem = KS % (int)gridDim.y, s = (int)blockIdx.y;
     k_first = s * per + min(s, rem);
@@ -124,12 +165,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
   // loads are unconditional (a guarded load is waited for at once): a unit past
   // the end re-reads the last one and is not multiplied
   auto load = [&](Unit& u, int c) __attribute__((always_inline)) {
-    const int64_t k = (int64_t)min(k_first + c, KS - 1) * 128;  // bytes
+    const int64_t k = (int64_t)min(k_first + c, KS - 1) * 128;  // bytes of b
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        u.v[t][h] = *(const u16x8_u*)(base[t < RT ? 0 : 1] + k + off[t][h]);
+        u.v[t][h] = *(const u16x8_u*)(base[t < RT ? 0 : 1] + (t < RT ? k : k * XS) + off[t][h]);
   };
   if (wave < NU) {
     Unit u0, u1;
@@ -143,18 +184,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
       if (c + NW < NU) multiply(u1);
     }
   }
-  // the last K % 64 elements, one wave (one with the fewest chunks)
+  // the last K % KU elements, one wave (one with the fewest units)
   if (has_tail && wave == NW - 1) {
-    const int64_t k0 = p.K / 64 * 64;
+    const int64_t k0 = p.K / KU * KU;
     Unit u;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const uint16_t* q = (const uint16_t*)(base[t < RT ? 0 : 1] + off[t][h]) + k0;
+        const char* q = base[t < RT ? 0 : 1] + off[t][h] + (t < RT ? k0 * BE : k0 * 2);
+        // k of the lane's first element, elements per 16-bit word
+        const int64_t k = k0 + (t < RT ? 16 / BE * (lane & 7) : 64 * ((t - RT) % XS) + 8 * (lane & 7));
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          u.v[t][h][e] = k0 + 8 * (lane & 7) + e < p.K ? q[e] : (uint16_t)0;
+        for (int e = 0; e < 8; ++e) {
+          if (I8 && t < RT) {
+            const uint16_t lo = k + 2 * e < p.K ? (uint8_t)q[2 * e] : 0;
+            const uint16_t hi = k + 2 * e + 1 < p.K ? (uint8_t)q[2 * e + 1] : 0;
+            u.v[t][h][e] = lo | (hi << 8);
+          } else {
+            u.v[t][h][e] = k + e < p.K ? ((const uint16_t*)q)[e] : (uint16_t)0;
+          }
+        }
       }
     multiply(u);
   }
@@ -180,27 +230,12 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
       *(f32x4_t*)(part + ((int64_t)blockIdx.y * p.M + m) * ldp + n) = s;
       continue;
     }
-    f32x4_t bb = {};
-    if constexpr (HAS_BIAS)
-      bb = load_col4_t<T>(p.bias, p.bias_dtype, n, p.bias_sn, p.N, m * p.bias_sm);
-    u16x4_t v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x = p.alpha * s[e];
-      if constexpr (HAS_BIAS) x += p.beta * bb[e];
-      v[e] = MfmaOp<T>::store(x);
-    }
-    uint16_t* dst = p.c + m * p.ldc + n;
-    if (n + 3 < p.N && (((uintptr_t)dst) & 7) == 0) {
-      *(u16x4_t*)dst = v;
-    } else {
-      for (int e = 0; e < 4 && n + e < p.N; ++e) dst[e] = v[e];
-    }
+    rows_store<T, HAS_BIAS, I8>(p, m, n, s);
   }
 }
 
 // out = alpha * sum_s part[s] + beta * bias, the slices added in order
-template <typename T, bool HAS_BIAS>
+template <typename T, bool HAS_BIAS, bool I8>
 __global__ __launch_bounds__(256) void rows_combine_kernel(GemmArgs p, const float* part, int S,
                                                            int64_t ldp) {
   const int64_t runs = ldp / 4;
@@ -211,25 +246,10 @@ __global__ __launch_bounds__(256) void rows_combine_kernel(GemmArgs p, const flo
   f32x4_t s = *(const f32x4_t*)src;
 #pragma unroll 8
   for (int i = 1; i < S; ++i) s += *(const f32x4_t*)(src + i * p.M * ldp);
-  f32x4_t bb = {};
-  if constexpr (HAS_BIAS)
-    bb = load_col4_t<T>(p.bias, p.bias_dtype, n, p.bias_sn, p.N, m * p.bias_sm);
-  u16x4_t v;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float x = p.alpha * s[e];
-    if constexpr (HAS_BIAS) x += p.beta * bb[e];
-    v[e] = MfmaOp<T>::store(x);
-  }
-  uint16_t* dst = p.c + m * p.ldc + n;
-  if (n + 3 < p.N && (((uintptr_t)dst) & 7) == 0) {
-    *(u16x4_t*)dst = v;
-  } else {
-    for (int e = 0; e < 4 && n + e < p.N; ++e) dst[e] = v[e];
-  }
+  rows_store<T, HAS_BIAS, I8>(p, m, n, s);
 }
 
-template <typename T, int MT, int RT, int NW, bool HB>
+template <typename T, int MT, int RT, int NW, bool HB, bool I8>
 mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
   const unsigned tiles = ceil_div_u(q.N, 16 * RT);
   const int64_t ldp = (q.N + 3) / 4 * 4;
@@ -239,15 +259,15 @@ mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
     S = 1;
   }
   if (S <= 1) {
-    hipLaunchKernelGGL((gemm_rows_kernel<T, MT, RT, NW, HB, false>), dim3(tiles), dim3(64 * NW),
+    hipLaunchKernelGGL((gemm_rows_kernel<T, MT, RT, NW, HB, false, I8>), dim3(tiles), dim3(64 * NW),
                        0, s, q, nullptr, (int64_t)0);
     return check_launch(what);
   }
   float* part = (float*)ws.get();
-  hipLaunchKernelGGL((gemm_rows_kernel<T, MT, RT, NW, false, true>), dim3(tiles, (unsigned)S),
+  hipLaunchKernelGGL((gemm_rows_kernel<T, MT, RT, NW, false, true, I8>), dim3(tiles, (unsigned)S),
                      dim3(64 * NW), 0, s, q, part, ldp);
   MI_RETURN_IF(check_launch(what));
-  hipLaunchKernelGGL((rows_combine_kernel<T, HB>), dim3(ceil_div_u(q.M * (ldp / 4), 256)),
+  hipLaunchKernelGGL((rows_combine_kernel<T, HB, I8>), dim3(ceil_div_u(q.M * (ldp / 4), 256)),
                      dim3(256), 0, s, q, (const float*)part, S, ldp);
   return check_launch(what);
 }
@@ -264,23 +284,40 @@ mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
 template <typename T, int MT, bool HB>
 mi_status_t pick_mt(const GemmArgs& q, hipStream_t s, const char* what) {
   if constexpr (MT == 1) {
-    return q.K <= 8192 ? launch<T, 1, 1, 16, HB>(q, 1, s, what)
-                       : launch<T, 1, 1, 8, HB>(q, 1, s, what);
+    if constexpr (!HB)
+      if (q.K <= 8192) return launch<T, 1, 1, 16, HB, false>(q, 1, s, what);
+    return launch<T, 1, 1, 8, HB, false>(q, 1, s, what);
   } else {
     const int64_t tiles = (q.N + 63) / 64;
-    if (tiles >= 128) return launch<T, MT, 4, 4, HB>(q, 1, s, what);
-    if (q.M * q.K < (1 << 18)) return launch<T, MT, 1, 8, HB>(q, 1, s, what);
-    return launch<T, MT, 4, 4, HB>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
+    if (tiles >= 128) return launch<T, MT, 4, 4, HB, false>(q, 1, s, what);
+    if (q.M * q.K < (1 << 18)) return launch<T, MT, 1, 8, HB, false>(q, 1, s, what);
+    return launch<T, MT, 4, 4, HB, false>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
   }
 }
 
+// The same for an int8 weight: half the bytes per element of b, so a's rows weigh
+// twice as much, but a unit's widening and four MFMAs per fragment favour small
+// blocks.  us: M8 N4096 K4224 10.8 -> 5.8, M15 N1920 K7123 106 -> 12.6, M24
+// N11008 K4224 28 -> 17 in blocks of 64 rows (19.5 in 16), M64 N4096 K4224 24 ->
+// 13 in 16 (16 sliced), M64 N4096 K8192 39 -> 19 sliced (22 in 16).
+template <typename T, int MT, bool HB>
+mi_status_t pick_mt8(const GemmArgs& q, hipStream_t s, const char* what) {
+  if constexpr (MT > 1) {
+    const int64_t tiles = (q.N + 63) / 64;
+    if (tiles >= 128) return launch<T, MT, 4, 4, HB, true>(q, 1, s, what);
+    if (q.M * q.K >= (1 << 19))
+      return launch<T, MT, 4, 4, HB, true>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
+  }
+  return launch<T, MT, 1, 8, HB, true>(q, 1, s, what);
+}
+
 template <typename T, bool HB>
-mi_status_t pick(const GemmArgs& q, hipStream_t s, const char* what) {
+mi_status_t pick(const GemmArgs& q, bool i8, hipStream_t s, const char* what) {
   switch ((q.M + 15) / 16) {
-    case 1: return pick_mt<T, 1, HB>(q, s, what);
-    case 2: return pick_mt<T, 2, HB>(q, s, what);
-    case 3: return pick_mt<T, 3, HB>(q, s, what);
-    default: return pick_mt<T, 4, HB>(q, s, what);
+    case 1: return i8 ? pick_mt8<T, 1, HB>(q, s, what) : pick_mt<T, 1, HB>(q, s, what);
+    case 2: return i8 ? pick_mt8<T, 2, HB>(q, s, what) : pick_mt<T, 2, HB>(q, s, what);
+    case 3: return i8 ? pick_mt8<T, 3, HB>(q, s, what) : pick_mt<T, 3, HB>(q, s, what);
+    default: return i8 ? pick_mt8<T, 4, HB>(q, s, what) : pick_mt<T, 4, HB>(q, s, what);
   }
 }
 
@@ -294,8 +331,9 @@ bool gemm_rows_eligible(const GemmArgs& q) {
 
 mi_status_t launch_gemm_rows(const GemmArgs& q, bool f16, bool has_bias, hipStream_t s,
                              const char* what) {
-  if (f16) return has_bias ? pick<F16, true>(q, s, what) : pick<F16, false>(q, s, what);
-  return has_bias ? pick<BF16, true>(q, s, what) : pick<BF16, false>(q, s, what);
+  const bool i8 = q.scale != nullptr;
+  if (f16) return has_bias ? pick<F16, true>(q, i8, s, what) : pick<F16, false>(q, i8, s, what);
+  return has_bias ? pick<BF16, true>(q, i8, s, what) : pick<BF16, false>(q, i8, s, what);
 }
 
 }  // namespace mi
