@@ -801,3 +801,18 @@ def test_copy_of_contiguous_rows(dtype, rows, width, pad_in, pad_out):
     _abi.copy_(dv, src.cuda()[:, :, pad_in:])
     dst[:, :, pad_out:] = sv
     assert torch.equal(ddst.cpu(), dst)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols", [(1, 9), (3, 200), (8, 8), (9, 65), (257, 1001), (64, 4099)])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_transposed_copy_edges(dtype, rows, cols, pad):
+    """Transposing copies around the 16-byte pieces, at odd leading dims and
+    offsets on both sides."""
+    gen = torch.Generator().manual_seed(rows)
+    src = torch.randint(-99, 99, (2, cols, rows + pad), generator=gen).to(dtype)
+    dst = torch.full((2, rows, cols + 3 * pad), 77).to(dtype)
+    ddst = dst.cuda()
+    _abi.copy_(ddst[:, :, pad:pad + cols], src.cuda()[:, :, pad:].transpose(1, 2))
+    dst[:, :, pad:pad + cols] = src[:, :, pad:].transpose(1, 2)
+    assert torch.equal(ddst.cpu(), dst)

@@ -253,9 +253,9 @@ __global__ __launch_bounds__(256) void transpose_kernel(T* __restrict__ out, con
 // go round robin to the 8 XCDs, so ids are renumbered to give each XCD one
 // contiguous range of tiles (neighbouring columns share its L2); measured on
 // a bf16 8192^2 transpose: 6.1 TB/s against 4.8 without the renumbering and
-// with non-temporal accesses.  Lanes whose block crosses the edge copy
-// element by element.  The host checks that both tensors and their leading
-// dims are 16-byte aligned.
+// with non-temporal accesses.  Addresses need only the element's alignment; a
+// block that would cross an edge is moved back inside (two lanes then write the
+// same values).  The host checks R, C >= E.
 constexpr int kTrWaves = 4;
 
 // Bijection of [0, n): the ids that land on one XCD become one range.
@@ -283,36 +283,35 @@ __global__ __launch_bounds__(64 * kTrWaves) void transpose_vec_kernel(
   const int a = lane & 7, b = lane >> 3;
   const unsigned id = xcd_contiguous(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
   const unsigned bx = id % gridDim.x, by = id / gridDim.x;
-  const int64_t r = ((int64_t)by * kTrWaves + wave) * (8 * E) + a * E;
-  const int64_t c = (int64_t)bx * (8 * E) + b * E;
+  const int64_t r0 = ((int64_t)by * kTrWaves + wave) * (8 * E) + a * E;
+  const int64_t c0 = (int64_t)bx * (8 * E) + b * E;
   const T* s = src + (int64_t)blockIdx.z * src_bs;
   T* o = out + (int64_t)blockIdx.z * out_bs;
-  if (r >= R || c >= C) return;
-  if (r + E <= R && c + E <= C) {
-    TrPiece<T> v[E], t[E];
+  if (r0 >= R || c0 >= C) return;
+  const int64_t r = min(r0, R - E), c = min(c0, C - E);
+  typedef u32x4_t __attribute__((aligned(2))) any_t;
+  TrPiece<T> v[E], t[E];
 #pragma unroll
-    for (int j = 0; j < E; ++j) v[j].v = *(const uint4*)(s + (c + j) * src_ld + r);
-    if constexpr (E == 8) {
-      // t[i].w[m] = (v[2m].e[i], v[2m+1].e[i]): the low or high halves of
-      // word i/2 of two column pieces
+  for (int j = 0; j < E; ++j)
+    v[j].v = __builtin_bit_cast(uint4, (u32x4_t)*(const any_t*)(s + (c + j) * src_ld + r));
+  if constexpr (E == 8) {
+    // t[i].w[m] = (v[2m].e[i], v[2m+1].e[i]): the low or high halves of
+    // word i/2 of two column pieces
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
-          t[i].w[m] = __builtin_amdgcn_perm(v[2 * m + 1].w[i >> 1], v[2 * m].w[i >> 1],
-                                            (i & 1) ? 0x07060302u : 0x05040100u);
-    } else {
+      for (int m = 0; m < 4; ++m)
+        t[i].w[m] = __builtin_amdgcn_perm(v[2 * m + 1].w[i >> 1], v[2 * m].w[i >> 1],
+                                          (i & 1) ? 0x07060302u : 0x05040100u);
+  } else {
 #pragma unroll
-      for (int i = 0; i < E; ++i)
+    for (int i = 0; i < E; ++i)
 #pragma unroll
-        for (int m = 0; m < E; ++m) t[i].e[m] = v[m].e[i];
-    }
-#pragma unroll
-    for (int i = 0; i < E; ++i) *(uint4*)(o + (r + i) * out_ld + c) = t[i].v;
-    return;
+      for (int m = 0; m < E; ++m) t[i].e[m] = v[m].e[i];
   }
-  for (int i = 0; i < E && r + i < R; ++i)
-    for (int j = 0; j < E && c + j < C; ++j) o[(r + i) * out_ld + c + j] = s[(c + j) * src_ld + r + i];
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+    *(any_t*)(o + (r + i) * out_ld + c) = __builtin_bit_cast(u32x4_t, t[i].v);
 }
 
 template <typename T>
@@ -329,8 +328,8 @@ __global__ __launch_bounds__(kBlock) void copy_raw_kernel(T* out, const T* src,
 // Rows that are contiguous in both operands (a padded or sliced matrix, rows of
 // any length and offset): 16-byte accesses at element alignment, four in flight
 // per lane; a row's last piece is moved back to end with the row, where two
-// lanes then write the same bytes.  Element by element such copies ran at 1.4
-// TB/s (bf16 [3840, 3443] into rows of 3448: 37 us).
+// lanes then write the same bytes.  bf16 [4615, 3443] into rows of 3448 takes 13 us
+// (37 element by element).
 __global__ __launch_bounds__(kBlock) void copy_rows_kernel(char* out, const char* src,
                                                            OffsetCalc<2> oc, int esz, int64_t len,
                                                            uint32_t pieces, int64_t total) {
@@ -773,8 +772,9 @@ mi_status_t mi_copy(const mi_tensor_t* out, const mi_tensor_t* src, mi_stream_t 
       const int64_t obs = nd == 3 ? it.strides[0][0] : 0, sbs = nd == 3 ? it.strides[1][0] : 0;
       const int64_t E = 16 / esz;
       const int64_t sld = it.strides[1][nd - 1], old_ = it.strides[0][nd - 2];
-      const bool vec_ok = ((uintptr_t)it.data[0] % 16) == 0 && ((uintptr_t)it.data[1] % 16) == 0 &&
-                          sld % E == 0 && old_ % E == 0 && obs % E == 0 && sbs % E == 0;
+      // (bf16 [4615, 3840] and [4615, 3443] at odd leading dims: 26 and 31 us by the LDS
+      // tiles)
+      const bool vec_ok = R >= E && C >= E;
       const dim3 vgrid(ceil_div_u(C, 8 * E), ceil_div_u(R, 8 * E * kTrWaves), (unsigned)batch);
       if (vec_ok && vgrid.y <= 65535) {
         if (esz == 2)
