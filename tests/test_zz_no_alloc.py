@@ -184,3 +184,34 @@ def test_noalloc_mean_captured_in_a_gcu_graph_replays_equal_eager():
     assert_exact(out.cpu(), torch.mean(x, 0).cpu(), "no-alloc mean replay with new input")
     assert_close(out, aten.mean(rn((16384, 4096), 9), 0), "fp32", "replay vs CPU ATen")
     graph.reset()
+
+
+def test_sliced_products_without_workspace():
+    """Products and attention that slice K (or the keys) into partial sums run
+    whole where the workspace allocator has nothing to give."""
+    cuda = lambda *s, dt=torch.bfloat16, seed=1: rn(s, seed, dt).cuda()
+    refused = _abi._ALLOC_FN(lambda nbytes, stream, ctx: None)
+    freed = _abi._FREE_FN(lambda ptr, stream, ctx: None)
+    _abi.check("mi_set_workspace_allocator", _abi.lib().mi_set_workspace_allocator(refused, freed, None))
+    try:
+        for M, N, K, dt in [(64, 1024, 8192, torch.bfloat16), (128, 2048, 4096, torch.float16),
+                            (42, 1216, 768, torch.float32)]:
+            a, b = cuda(M, K, dt=dt), cuda(N, K, dt=dt, seed=2)
+            out = torch.empty(M, N, dtype=dt, device="cuda")
+            _abi.mm(out, a, b.t())
+            ref = aten.addmm(None, a.cpu(), b.cpu().t(), beta=0.0)
+            assert_close(out, ref, "fp32" if dt == torch.float32 else "bf16", f"mm {M}x{N}x{K}")
+        w = torch.randint(-127, 127, (1000, 1024), dtype=torch.int8)
+        sc = torch.full((1000,), 0.01)
+        for M in (64, 100, 600):
+            x = cuda(M, 1024, seed=3)
+            out = torch.empty(M, 1000, dtype=torch.bfloat16, device="cuda")
+            _abi.int8_linear(out, x, w.cuda(), sc.cuda())
+            assert_close(out, aten.int8_linear(x.cpu(), w, sc), "bf16", f"int8 {M}")
+        q, k, v = cuda(1, 8, 1, 128), cuda(1, 2, 3000, 128, seed=4), cuda(1, 2, 3000, 128, seed=5)
+        out, lse = torch.empty_like(q), torch.empty(1, 8, 1, device="cuda")
+        _abi.flash_attention_fwd(out, lse, q, k, v, False)
+        assert_close(out, aten.sdpa(q.cpu(), k.cpu(), v.cpu(), False)[0], "bf16", "attention")
+        torch.cuda.synchronize()
+    finally:
+        torch_gcu._C._register_library_workspace()

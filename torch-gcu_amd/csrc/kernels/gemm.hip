@@ -1009,7 +1009,11 @@ mi_status_t launch_mfma(const GemmArgs& q, int64_t batch, hipStream_t s, const c
   // tiles x 2: 75 us against 107), else 128-row tiles sized to the CUs
   if (I8 && batch == 1 && q.M > 64 && dl_eligible(q, true)) {
     const int S = splitk_slices(q);
-    if (S > 1) return launch_splitk<T, HB, true>(q, S, s, what);
+    if (S > 1) {
+      const mi_status_t st = launch_splitk<T, HB, true>(q, S, s, what);
+      if (st != MI_ERR_WORKSPACE && st != MI_ERR_TOO_LARGE) return st;
+      clear_error();  // no room for the partial sums: the whole K in one block
+    }
     if (q.M <= 4 * mid::BM) return launch_mid<T, HB>(q, s, what);
   }
   if constexpr (!I8) {
