@@ -404,3 +404,26 @@ def test_causal_attention_head_groups(B, H, Hk, S, D):
     err = (out.cpu().double() - torch.from_numpy(ref).double()).abs()
     assert bool((err <= bound).all()), (err / bound).max()
     assert (lse.cpu().double() - torch.from_numpy(ref_lse).double()).abs().max().item() < 1e-3
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-40])
+@pytest.mark.parametrize("B,H,Hk,Sq,Sk,D,causal", [
+    (1, 2, 2, 130, 130, 128, True), (1, 2, 2, 130, 201, 64, False),  # the tiled kernel
+    (1, 8, 2, 1, 1001, 128, False), (2, 4, 1, 3, 4100, 64, False),   # the key-split one
+])
+def test_attention_zero_scale(scale, B, H, Hk, Sq, Sk, D, causal):
+    """A scale of zero (or one that a float flushes) is the mean of the visible
+    values: masked keys and the keys past a ragged last tile stay masked."""
+    q, k, v = rn((B, H, Sq, D), 94), rn((B, Hk, Sk, D), 95), rn((B, Hk, Sk, D), 96)
+    out = torch.empty(B, H, Sq, D, dtype=torch.bfloat16, device="cuda")
+    lse = torch.empty(B, H, Sq, device="cuda")
+    _abi.flash_attention_fwd(out, lse, q.cuda(), k.cuda(), v.cuda(), causal, scale)
+    ref, ref_lse = npr.attention64(q.float().numpy(), k.float().numpy(), v.float().numpy(), causal, scale)
+    mag, _ = npr.attention64(q.float().numpy(), k.float().numpy(), abs(v.float().numpy()), causal, scale)
+    # weights of 1 are exact in bf16, so the output's rounding alone (8 significant
+    # bits: half an ulp is at most 2^-8 of it) and fp32 sums of Sk terms (Sk 2^-24
+    # of their magnitudes)
+    bound = 1.01 * 2.0 ** -8 * torch.from_numpy(abs(ref)) + Sk * 2.0 ** -24 * torch.from_numpy(mag) + 1e-6
+    err = (out.cpu().double() - torch.from_numpy(ref)).abs()
+    assert bool((err <= bound).all()), (err / bound).max()
+    assert (lse.cpu().double() - torch.from_numpy(ref_lse)).abs().max().item() < 1e-5

@@ -34,6 +34,7 @@
 // interleaved longest first, the group as large as its K and V fit the L2: head
 // by head, each head's longest tile started late and the last ones ran alone.
 #include <algorithm>
+#include <cfloat>
 
 #include "attention_common.h"
 
@@ -540,7 +541,11 @@ extern "C" mi_status_t mi_flash_attention_fwd(const mi_tensor_t* out, const mi_t
   MI_CHECK_ARG(Sk * k->strides[2] + D < 0x7fffffffLL && Sk * v->strides[2] + D < 0x7fffffffLL &&
                    Sq + QT < 0x7fffffffLL,
                "attention: a (batch, head) of k or v spans more than 2^31 elements");
+  // a masked key's raw score is infinite, and its product with a zero scale would
+  // be NaN: below the smallest normal float the scale is that float, which leaves
+  // masked keys infinite and any finite score of ordinary size without weight
   a.scale_log2 = (float)(scale * 1.4426950408889634);
+  if (std::fabs(a.scale_log2) < FLT_MIN) a.scale_log2 = std::copysign(FLT_MIN, a.scale_log2);
   a.causal = is_causal ? 1 : 0;
   a.q_tiles = (int)((Sq + QT - 1) / QT);
   const int64_t nb = (int64_t)a.q_tiles * H * B;
