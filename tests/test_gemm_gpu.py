@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import aten
-from oracle.tolerance import assert_close
+from oracle.tolerance import assert_close, assert_exact
 from torch_gcu import _abi
 
 pytestmark = pytest.mark.gpu
@@ -642,3 +642,24 @@ def test_int8_linear_any_k(M, N, K, dtype, bias):
         _abi.int8_linear(out[:, :N], x.cuda(), wd, sc.cuda(), None if b is None else b.cuda())
         assert_close(out[:, :N], ref, "bf16", f"int8 {M}x{N}x{K}")
         assert bool((out[:, N] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 520, 1024), (8, 4096, 4096), (33, 1000, 257), (64, 8192, 1024)])
+def test_int8_few_rows_strided(M, N, K):
+    """Few rows with x, the weight or the output strided along the wrong
+    dimension: after the dense copies these are the dense call, so they take its
+    kernel and give its bits."""
+    x = rn((M, K), 100, torch.bfloat16, 1.0).cuda()
+    w = torch.randint(-127, 128, (N, K), generator=g(101), dtype=torch.int8).cuda()
+    sc = (torch.rand(N, generator=g(102)) * 0.009 + 0.001).cuda()
+    dense = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    _abi.int8_linear(dense, x, w, sc)
+    wide = torch.zeros(M, 2 * K, dtype=torch.bfloat16, device="cuda")
+    wide[:, ::2] = x
+    for name, xs, ws, out in [
+            ("x transposed", x.t().contiguous().t(), w, torch.empty_like(dense)),
+            ("x every other column", wide[:, ::2], w, torch.empty_like(dense)),
+            ("weight transposed", x, w.t().contiguous().t(), torch.empty_like(dense)),
+            ("out transposed", x, w, torch.empty(N, M, dtype=dense.dtype, device="cuda").t())]:
+        _abi.int8_linear(out, xs, ws, sc)
+        assert_exact(out, dense, f"{M}x{N}x{K} {name}")

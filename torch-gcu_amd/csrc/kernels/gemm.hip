@@ -1202,20 +1202,20 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
   // or B as row-major [K, N] rows read in place by the large-tile kernel
   Workspace wa, wb, wc;
   Mat Bt = transposed(B);
-  // few rows: the weight stream kernels, operands read as they are.  An int8
-  // weight of whole 1 KiB slabs keeps int8_stream_kernel where its N / CUs rows
-  // per block are worth its 48-row slabs (M24 N11008 K4096 14.1 us against 16.4;
-  // M8 N4096 K4096 8.1 against 6.7, M64 N4096 K8192 39 against 19)
-  const bool stream8 = int8 && M <= 64 && K % kStSlab == 0 && N >= 32 * cu_count() && A.s1 == 1 &&
-                       (A.s0 % 8 == 0 || M == 1) && Bt.s1 == 1 && Bt.s0 % 16 == 0 &&
-                       ((((uintptr_t)A.data) | ((uintptr_t)B.data)) & 15) == 0 &&
-                       (C.s1 == 1 || N == 1);
-  if (!stream8 && batch == 1 && M <= kRowsMax && (A.s1 == 1 || K == 1) && (Bt.s1 == 1 || K == 1) &&
-      (C.s1 == 1 || N == 1)) {
+  // Few rows: the weight stream kernels.  An int8 weight of whole 1 KiB slabs
+  // keeps int8_stream_kernel where its N / CUs rows per block are worth its 48-row
+  // slabs (M24 N11008 K4096 14.1 us against 16.4; M8 N4096 K4096 8.1 against 6.7,
+  // M64 N4096 K8192 39 against 19).  Asked of the operands as they are, and for
+  // int8 of the dense copies where those were needed (M8 N4096 K4096, x at a column
+  // stride of 2: 46 us on the large-M tiles, 9 so).
+  auto few_rows = [&](const Mat& a, const Mat& bt, const Mat& c, mi_status_t* st) {
+    if (batch != 1 || M > kRowsMax || (a.s1 != 1 && K != 1) || (bt.s1 != 1 && K != 1) ||
+        (c.s1 != 1 && N != 1))
+      return false;
     GemmArgs q{};
-    q.a = (const uint16_t*)A.data;
-    q.b = B.data;
-    q.c = (uint16_t*)C.data;
+    q.a = (const uint16_t*)a.data;
+    q.b = bt.data;
+    q.c = (uint16_t*)c.data;
     q.bias = bv.data;
     q.bias_dtype = bv.dtype;
     q.bias_sm = bv.sm;
@@ -1223,15 +1223,25 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
     q.M = M;
     q.N = N;
     q.K = K;
-    q.lda = A.s0;
-    q.ldb = Bt.s0;
-    q.ldc = C.s0;
+    q.lda = a.s0;
+    q.ldb = bt.s0;
+    q.ldc = c.s0;
     q.scale = int8 ? (const float*)scale->data : nullptr;
     q.alpha = (float)alpha;
     q.beta = (float)beta;
-    if (gemm_rows_eligible(q))
-      return launch_gemm_rows(q, A.dtype == MI_F16, has_bias, stream, what);
-  }
+    const bool f16 = a.dtype == MI_F16;
+    if (int8 && K % kStSlab == 0 && N >= 32 * cu_count() && (q.lda % 8 == 0 || M == 1) &&
+        q.ldb % 16 == 0 && ((((uintptr_t)q.a) | ((uintptr_t)q.b)) & 15) == 0) {
+      if (f16) *st = has_bias ? launch_stream<F16, true>(q, stream) : launch_stream<F16, false>(q, stream);
+      else *st = has_bias ? launch_stream<BF16, true>(q, stream) : launch_stream<BF16, false>(q, stream);
+      return true;
+    }
+    if (!gemm_rows_eligible(q)) return false;
+    *st = launch_gemm_rows(q, f16, has_bias, stream, what);
+    return true;
+  };
+  mi_status_t few_st;
+  if (few_rows(A, Bt, C, &few_st)) return few_st;
   MI_RETURN_IF(dense_rows(A, wa, stream));
   bool b_kn = false;
   if (!int8 && B.s1 == 1 && N > 1 && Bt.s1 != 1) {
@@ -1293,13 +1303,8 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
     }
     return MI_OK;
   }
-  if (stream8) {
-    mi_status_t st;
-    if (A.dtype == MI_BF16)
-      st = has_bias ? launch_stream<BF16, true>(q, stream) : launch_stream<BF16, false>(q, stream);
-    else
-      st = has_bias ? launch_stream<F16, true>(q, stream) : launch_stream<F16, false>(q, stream);
-    MI_RETURN_IF(st);
+  if (int8 && few_rows(A, Bt, Cw, &few_st)) {
+    MI_RETURN_IF(few_st);
   } else if (A.dtype == MI_BF16) {
     MI_RETURN_IF(dispatch_mfma<BF16>(q, int8, has_bias, batch, stream, what));
   } else {
