@@ -816,3 +816,43 @@ def test_transposed_copy_edges(dtype, rows, cols, pad):
     _abi.copy_(ddst[:, :, pad:pad + cols], src.cuda()[:, :, pad:].transpose(1, 2))
     dst[:, :, pad:pad + cols] = src[:, :, pad:].transpose(1, 2)
     assert torch.equal(ddst.cpu(), dst)
+
+
+@pytest.mark.parametrize("width", [1, 31, 64, 65, 128])
+def test_short_rows_sum_an_element_per_lane(width):
+    """Rows of up to 128 elements are summed one element per lane and the lanes
+    by halves, whatever the addresses: bit for bit that order."""
+    x = torch.randn(1001, width, generator=g(width))
+    buf = torch.empty(x.numel() + 1, device=DEV)
+    buf[1:].copy_(x.reshape(-1))
+    lanes = torch.zeros(1001, 64)
+    for j in range(0, width, 64):
+        part = x[:, j:j + 64]
+        lanes[:, :part.shape[1]] += part
+    for off in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, torch.arange(64) ^ off]
+    for xd in (dev(x), buf[1:].view(x.shape)):
+        s = torch.empty(1001, device=DEV)
+        _abi.sum_(s, xd, [-1])
+        assert_exact(s, lanes[:, 0], f"sum {width}")
+
+
+@pytest.mark.parametrize("dtype", [torch.int8, torch.bfloat16, torch.int32])
+@pytest.mark.parametrize("width", [127, 128, 129, 255, 511, 512, 513, 514])
+def test_row_reductions_around_the_vector_widths(dtype, width):
+    """Either side of the lengths from which rows take 16-byte loads, the
+    remainder's lanes included, at both address classes (values whose sums
+    are exact in every type)."""
+    x = torch.randint(0, 3, (70, width), generator=g(width)).to(dtype)
+    buf = torch.empty(x.numel() + 1, dtype=dtype, device=DEV)
+    buf[1:].copy_(x.reshape(-1))
+    x[:, -1] = 7  # the last element is the max
+    buf[1:].view(x.shape)[:, -1] = 7
+    for xd in (dev(x), buf[1:].view(x.shape)):
+        m = torch.empty(70, dtype=dtype, device=DEV)
+        _abi.amax(m, xd, [-1])
+        assert_exact(m, x.amax(-1), f"amax {width}")
+        sd = torch.float32 if dtype == torch.bfloat16 else torch.int64
+        s = torch.empty(70, dtype=sd, device=DEV)
+        _abi.sum_(s, xd, [-1])
+        assert_exact(s, x.sum(-1, dtype=sd), f"sum {width}")

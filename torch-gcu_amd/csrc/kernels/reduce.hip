@@ -176,57 +176,73 @@ __global__ __launch_bounds__(kRowBlock) void row_reduce_kernel(
   }
 }
 
-// Many short rows: one wave per row, four 16-byte loads in flight per lane
-// (unconditional, as above), then the remainder element by element.
-template <typename Tag, bool MX>
+// One wave per row.  VECS: four 16-byte loads in flight per lane and the
+// remainder's element (unconditional, as above); else an element per lane at a
+// time, for rows that give few lanes a 16-byte load.
+template <typename Tag, bool MX, bool VECS>
 __global__ __launch_bounds__(256) void row_reduce_wave_kernel(
     const typename RT<Tag>::storage* __restrict__ in, int64_t rows, int64_t R,
     int64_t row_stride, int op, RedOut out) {
   typedef typename RT<Tag>::storage St;
   typedef typename RT<Tag>::acc A;
-  constexpr int VEC = 16 / sizeof(St) > 0 ? 16 / sizeof(St) : 1, U = 4;
+  constexpr int VEC = 16 / sizeof(St), U = 4;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
   const St* p = in + row * row_stride;
   A acc = red_ident<A>(op);
-  union V {
-    uint4 u;
-    St s[VEC];
-  };
-  const int64_t nv = R / VEC;
-  for (int64_t v0 = lane; v0 < nv; v0 += 64 * U) {
-    V x[U];
-    bool ok[U];
+  if constexpr (VECS) {
+    union V {
+      uint4 u;
+      St s[VEC];
+    };
+    const int64_t nv = R / VEC;
+    const bool rem = lane < (int)(R - nv * VEC);
+    const St last = p[rem ? nv * VEC + lane : R - 1];
+    for (int64_t v0 = lane; v0 < nv; v0 += 64 * U) {
+      V x[U];
+      bool ok[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      ok[u] = v0 + 64 * u < nv;
-      x[u] = ld_stream_any<St, V>(p + (ok[u] ? v0 + 64 * u : nv - 1) * VEC);
-    }
+      for (int u = 0; u < U; ++u) {
+        ok[u] = v0 + 64 * u < nv;
+        x[u] = ld_stream_any<St, V>(p + (ok[u] ? v0 + 64 * u : nv - 1) * VEC);
+      }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (ok[u]) {
+      for (int u = 0; u < U; ++u) {
+        if (ok[u]) {
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) acc = red_comb<MX>(acc, RT<Tag>::load(x[u].s[e]));
+          for (int e = 0; e < VEC; ++e) acc = red_comb<MX>(acc, RT<Tag>::load(x[u].s[e]));
+        }
       }
     }
+    if (rem) acc = red_comb<MX>(acc, RT<Tag>::load(last));
+  } else {
+    for (int64_t j = lane; j < R; j += 64) acc = red_comb<MX>(acc, RT<Tag>::load(p[j]));
   }
-  for (int64_t j = nv * VEC + lane; j < R; j += 64)
-    acc = red_comb<MX>(acc, RT<Tag>::load(p[j]));
   acc = wave_red(op, acc);
   if (lane == 0) red_store(out, op, row, acc);
 }
 
+// 16-byte loads above 128 elements a row (us, by elements and in vectors: bf16
+// [1000000, 31] 141 and 261, [1000000, 128] 179 and 228, [100000, 200] 28 and 25;
+// f32 [1000000, 64] 141 and 211), or above 512 where 1- and 2-byte rows start at
+// odd addresses (bf16 at an offset of one, [20000, 512] 8.2 and 11.0).
 template <typename Tag>
 void launch_row_wave(const typename RT<Tag>::storage* in, int64_t rows, int64_t R, int op, RedOut o,
                      hipStream_t stream) {
   const dim3 grid(ceil_div_u(rows, 4)), block(256);
-  if (op == R_MAX)
-    hipLaunchKernelGGL((row_reduce_wave_kernel<Tag, true>), grid, block, 0, stream, in, rows, R, R,
-                       op, o);
-  else
-    hipLaunchKernelGGL((row_reduce_wave_kernel<Tag, false>), grid, block, 0, stream, in, rows, R, R,
-                       op, o);
+  const bool words = (((uintptr_t)in | (uintptr_t)(R * sizeof(*in))) & 3) == 0;
+  auto run = [&](auto mx, auto vecs) {
+    hipLaunchKernelGGL((row_reduce_wave_kernel<Tag, decltype(mx)::value, decltype(vecs)::value>), grid,
+                       block, 0, stream, in, rows, R, R, op, o);
+  };
+  if (R > (words ? 128 : 512)) {
+    if (op == R_MAX) run(std::true_type(), std::true_type());
+    else run(std::false_type(), std::true_type());
+  } else {
+    if (op == R_MAX) run(std::true_type(), std::false_type());
+    else run(std::false_type(), std::false_type());
+  }
 }
 
 constexpr int kColUnroll = 4;  // rows a batch for narrow loads (two batches in flight)
