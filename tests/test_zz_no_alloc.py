@@ -215,3 +215,20 @@ def test_sliced_products_without_workspace():
         torch.cuda.synchronize()
     finally:
         torch_gcu._C._register_library_workspace()
+
+
+def test_int8_linear_above_512_rows_slices_where_it_pays():
+    """K slices over 256 x 256 tiles need workspace, 128 x 64 tiles over the whole
+    K none: short products run whole, long ones sliced, with the same result."""
+    gen = torch.Generator().manual_seed(12)
+    for M, N, K, slices in [(513, 256, 256, 0), (600, 1024, 1024, 0), (2000, 2048, 1024, 0),
+                            (600, 1024, 8192, 1), (2000, 1024, 4096, 1)]:
+        x = rn((M, K), M, torch.bfloat16)
+        w = torch.randint(-127, 128, (N, K), generator=gen, dtype=torch.int8)
+        sc = torch.rand(N, generator=gen) * 0.009 + 0.001
+        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        with CountingWorkspace() as ws:
+            _abi.int8_linear(out, x.cuda(), w.cuda(), sc.cuda())
+            torch.cuda.synchronize()
+            assert ws.allocs == slices, (M, N, K, ws.allocs)
+        assert_close(out, aten.int8_linear(x, w, sc), "bf16", f"int8 {M}x{N}x{K}")

@@ -970,6 +970,20 @@ int splitk_slices(const GemmArgs& q) {
   return s >= 2 ? (int)std::min<int64_t>(s, 16) : 1;
 }
 
+// Above 512 rows the slices have to beat 128 x 64 tiles over the whole K, by cost
+// in us: those take 0.42 us a K step, 0.7 where K is long, or 0.45 per block and
+// CU; a slice 1.3 us a step, and its partial sums go through the caches.  A fit to
+// 356 shapes (M 513 .. 4096, N 256 .. 8192, K 64 .. 8192; 0.7 % from the faster of
+// the two on average, 8 % at worst): M600 N1024 K1024 12.4 us whole, 25.5 in 16
+// slices; M2000 N1024 K4096 48.2 and 42.2; M3500 N2048 K4096 108 and 77.
+bool slices_pay(const GemmArgs& q, int S) {
+  const int64_t blocks = ((q.M + 127) / 128) * ((q.N + 63) / 64), steps = q.K / dl::BK;
+  const float step = std::max(q.K <= 2240 ? 0.42f : 0.7f, 0.45f * (float)blocks / (float)cu_count());
+  const float sliced = 14.f + 1.3f * (float)((steps + S - 1) / S) +
+                       (float)S * (float)q.M * (float)q.N * (8.f / 8.5e6f);
+  return sliced < 5.f + step * (float)steps;
+}
+
 template <typename T, bool HB>
 mi_status_t combine(const GemmArgs& q, const float* part, int S, int64_t ldp, hipStream_t s,
                     const char* what) {
@@ -1009,7 +1023,7 @@ mi_status_t launch_mfma(const GemmArgs& q, int64_t batch, hipStream_t s, const c
   // tiles x 2: 75 us against 107), else 128-row tiles sized to the CUs
   if (I8 && batch == 1 && q.M > 64 && dl_eligible(q, true)) {
     const int S = splitk_slices(q);
-    if (S > 1) {
+    if (S > 1 && (q.M <= 4 * mid::BM || slices_pay(q, S))) {
       const mi_status_t st = launch_splitk<T, HB, true>(q, S, s, what);
       if (st != MI_ERR_WORKSPACE && st != MI_ERR_TOO_LARGE) return st;
       clear_error();  // no room for the partial sums: the whole K in one block
