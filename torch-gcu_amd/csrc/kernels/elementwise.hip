@@ -326,14 +326,14 @@ __global__ __launch_bounds__(kBlock) void copy_raw_kernel(T* out, const T* src,
 }
 
 // Rows that are contiguous in both operands (a padded or sliced matrix, rows of
-// any length and offset): 16-byte accesses at element alignment, four in flight
-// per lane; a row's last piece is moved back to end with the row, where two
-// lanes then write the same bytes.  bf16 [4615, 3443] into rows of 3448 takes 13 us
+// any length and offset): 16-byte accesses at element alignment, U in flight per
+// lane; a row's last piece is moved back to end with the row, where two lanes
+// then write the same bytes.  bf16 [4615, 3443] into rows of 3448 takes 13 us
 // (37 element by element).
+template <int U>
 __global__ __launch_bounds__(kBlock) void copy_rows_kernel(char* out, const char* src,
                                                            OffsetCalc<2> oc, int esz, int64_t len,
                                                            uint32_t pieces, int64_t total) {
-  constexpr int U = 4;
   const int64_t i0 = (int64_t)blockIdx.x * (kBlock * U) + threadIdx.x;
   typedef u32x4_t __attribute__((aligned(1))) any_t;
   u32x4_t v[U];
@@ -807,8 +807,13 @@ mi_status_t mi_copy(const mi_tensor_t* out, const mi_tensor_t* src, mi_stream_t 
       oc.ndim = nd - 1;  // the rows
       const int64_t pieces = (len + 15) / 16, total = it.numel / it.sizes[nd - 1] * pieces;
       if (total <= (int64_t)kBlock * 4 * 0x7fffffff) {
-        hipLaunchKernelGGL(copy_rows_kernel, dim3(ceil_div_u(total, kBlock * 4)), dim3(kBlock), 0,
-                           stream, it.data[0], it.data[1], oc, esz, len, (uint32_t)pieces, total);
+        // four pieces a lane only where that leaves blocks for every CU
+        if (total > (int64_t)kBlock * 4 * cu_count())
+          hipLaunchKernelGGL(copy_rows_kernel<4>, dim3(ceil_div_u(total, kBlock * 4)), dim3(kBlock), 0,
+                             stream, it.data[0], it.data[1], oc, esz, len, (uint32_t)pieces, total);
+        else
+          hipLaunchKernelGGL(copy_rows_kernel<1>, dim3(ceil_div_u(total, kBlock)), dim3(kBlock), 0,
+                             stream, it.data[0], it.data[1], oc, esz, len, (uint32_t)pieces, total);
         return check_launch("copy_rows");
       }
     }
