@@ -663,3 +663,20 @@ def test_int8_few_rows_strided(M, N, K):
             ("out transposed", x, w, torch.empty(N, M, dtype=dense.dtype, device="cuda").t())]:
         _abi.int8_linear(out, xs, ws, sc)
         assert_exact(out, dense, f"{M}x{N}x{K} {name}")
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (33, 5, 9), (5, 33, 40), (64, 31, 1), (31, 64, 17), (65, 97, 33)])
+@pytest.mark.parametrize("lay", ["nn", "nt", "tn", "tt"])
+def test_f32_small_batches(M, N, K, lay):
+    """fp32 tiles that a product does not fill: pieces of an operand, waves and
+    chunks of the last step that lie outside are left out."""
+    a, b = torch.randn(300, M, K, generator=g(110)), torch.randn(300, K, N, generator=g(111))
+    da = a.cuda() if lay[0] == "n" else a.transpose(1, 2).contiguous().cuda().transpose(1, 2)
+    db = b.cuda() if lay[1] == "n" else b.transpose(1, 2).contiguous().cuda().transpose(1, 2)
+    out = torch.full((300, M, N + 1), 7.0, device="cuda")
+    _abi.bmm(out[:, :, :N], da, db)
+    ref = a.double() @ b.double()
+    # each of the K products and adds rounds once: K + 1 half ulps of the magnitudes
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ b.double().abs())
+    assert bool(((out[:, :, :N].cpu().double() - ref).abs() <= bound).all())
+    assert bool((out[:, :, N] == 7.0).all())
