@@ -680,3 +680,21 @@ def test_f32_small_batches(M, N, K, lay):
     bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ b.double().abs())
     assert bool(((out[:, :, :N].cpu().double() - ref).abs() <= bound).all())
     assert bool((out[:, :, N] == 7.0).all())
+
+
+@pytest.mark.parametrize("K", [5, 8, 9, 10, 11, 12, 13, 14, 15, 31, 60, 66, 79, 135])
+def test_bmm_k_remainders(K):
+    """Every remainder of K by 8, below and above a whole 64-wide step, of
+    operands that need no copy (a leading dim that is a multiple of 8)."""
+    a, b = rn((9, 100, K), 120, torch.bfloat16, 1.0), rn((9, 70, K), 121, torch.bfloat16, 1.0)
+    ld = (K + 7) // 8 * 8
+
+    def padded(t):  # NaN beyond the row's K elements
+        buf = torch.full((*t.shape[:2], ld), float("nan"), dtype=t.dtype, device="cuda")
+        buf[:, :, :K] = t.cuda()
+        return buf[:, :, :K]
+
+    out = torch.empty(9, 100, 70, dtype=torch.bfloat16, device="cuda")
+    _abi.bmm(out, padded(a), padded(b).transpose(1, 2))
+    ref = torch.stack([aten.addmm(None, x, y.t(), beta=0.0) for x, y in zip(a, b)])
+    assert_close(out, ref, "bf16", f"bmm K {K}")
