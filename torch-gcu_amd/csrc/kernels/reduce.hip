@@ -198,7 +198,8 @@ __global__ __launch_bounds__(256) void row_reduce_wave_kernel(
     };
     const int64_t nv = R / VEC;
     const bool rem = lane < (int)(R - nv * VEC);
-    const St last = p[rem ? nv * VEC + lane : R - 1];
+    St last = {};
+    if (nv * VEC < R) last = p[rem ? nv * VEC + lane : R - 1];
     for (int64_t v0 = lane; v0 < nv; v0 += 64 * U) {
       V x[U];
       bool ok[U];
