@@ -698,3 +698,29 @@ def test_bmm_k_remainders(K):
     _abi.bmm(out, padded(a), padded(b).transpose(1, 2))
     ref = torch.stack([aten.addmm(None, x, y.t(), beta=0.0) for x, y in zip(a, b)])
     assert_close(out, ref, "bf16", f"bmm K {K}")
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16 bias", "int8"])
+@pytest.mark.parametrize("M,N,K", [(1, 8192, 40), (16, 8197, 64), (3, 10250, 512), (16, 10241, 193),
+                                   (2, 8200, 513), (7, 8192, 1024), (1, 8193, 1025), (64, 200, 128), (33, 1000, 40)])
+def test_few_rows_short_k(kind, M, N, K):
+    """Short K with many weight rows: the launch shapes on either side of their
+    limits in N and K, ragged last blocks."""
+    dtype = torch.float16 if kind == "f16 bias" else torch.bfloat16
+    x = rn((M, K), 130, dtype, 1.0)
+    out = torch.full((M, N + 1), 7.0, dtype=dtype, device="cuda")
+    if kind == "int8":
+        w = torch.randint(-127, 128, (N, K), generator=g(131), dtype=torch.int8)
+        sc = torch.rand(N, generator=g(132)) * 0.009 + 0.001
+        _abi.int8_linear(out[:, :N], x.cuda(), w.cuda(), sc.cuda())
+        ref = aten.int8_linear(x, w, sc)
+    else:
+        w = rn((N, K), 131, dtype, 1.0)
+        bias = rn((N,), 132, dtype, 1.0) if kind == "f16 bias" else None
+        if bias is None:
+            _abi.mm(out[:, :N], x.cuda(), w.cuda().t())
+        else:
+            _abi.addmm(out[:, :N], bias.cuda(), x.cuda(), w.cuda().t())
+        ref = aten.addmm(bias, x, w.t(), beta=0.0 if bias is None else 1.0)
+    assert_close(out[:, :N], ref, "bf16", f"{kind} {M}x{N}x{K}")
+    assert bool((out[:, N] == 7.0).all())

@@ -1250,6 +1250,11 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
       else *st = has_bias ? launch_stream<BF16, true>(q, stream) : launch_stream<BF16, false>(q, stream);
       return true;
     }
+    // (a short K is over before the waves that share it have paid: M64 N128256 K64
+    // 16.4 us here, 10.0 on the tiles of gemm_mid.hip; int8 M64 N28672 K320 12.2 and
+    // 9.1 on 128 x 64 ones)
+    if (!int8 && M > 32 && K <= 128 && gemm_mid_eligible(q)) return false;
+    if (int8 && M > 32 && K <= 768 && N >= 64 * cu_count()) return false;
     if (!gemm_rows_eligible(q)) return false;
     *st = launch_gemm_rows(q, f16, has_bias, stream, what);
     return true;

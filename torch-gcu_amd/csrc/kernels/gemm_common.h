@@ -98,6 +98,16 @@ __device__ __forceinline__ typename MfmaOp<T>::vec widen8(u32x2_t w) {
   return __builtin_bit_cast(typename MfmaOp<T>::vec, r);
 }
 
+// v's 16 bytes shifted down by `back` bytes, zeros behind: with the 16 bytes that
+// end with a row, the row's remainder as a chunk (back >= 16: a chunk past the row)
+typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u64x2_t shift_down(u64x2_t v, int back) {
+  const int s = 8 * (back & 7);
+  u64x2_t r = {v[0] >> s | (v[1] << 1) << (63 - s), v[1] >> s};
+  if (back & 8) r = u64x2_t{r[1], 0};
+  return back < 16 ? r : u64x2_t{};
+}
+
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
 

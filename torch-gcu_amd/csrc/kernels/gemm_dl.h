@@ -430,38 +430,36 @@ __global__ __launch_bounds__(C::NT, 2) void gemm_dl_kernel(GemmArgs p, float* pa
       const uint16_t* B0 = (const uint16_t*)p.b + batch * p.sb;
       // the copies' layout: LDS chunk lane % CH of a row holds global chunk
       // dl_swz(row, lane % CH); loads past K re-read inside the row
-      auto get = [&](int q) __attribute__((always_inline)) {
-        const bool is_a = q < NQA;
-        const int row = (is_a ? wave * NQA + q : wave * NQB + q - NQA) * RPK + lane / CH;
-        const uint16_t* src = is_a ? A0 + (int64_t)min(m0 + row, M - 1) * p.lda
-                                   : B0 + (int64_t)min(n0 + row, N - 1) * p.ldb;
-        const int k = kt0 + 8 * dl_swz(row, lane % CH);
-        u16x8_t v;
-        if (K % 8 == 0) {
-          v = *(const u16x8_t*)(src + min(k, K - 8));
-          if (k >= K) v = u16x8_t{};
-        } else if (K >= 8) {
-          // the row's last 8 elements, shifted down where the chunk passes K (M1500
-          // N1000 K130 12.3 us; 14.7 with a load per element)
-          typedef uint64_t u64x2_t __attribute__((ext_vector_type(2)));
-          typedef u64x2_t __attribute__((aligned(2))) u64x2_u;
-          const int kk = min(k, K - 8), sh = 16 * (k - kk);
-          const u64x2_t w = *(const u64x2_u*)(src + kk);
-          u64x2_t r = w;
-          if (sh >= 64) r = u64x2_t{w[1] >> (sh & 63), 0};
-          else if (sh > 0) r = u64x2_t{(w[0] >> sh) | (w[1] << (64 - sh)), w[1] >> sh};
-          v = k >= K ? u16x8_t{} : __builtin_bit_cast(u16x8_t, r);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = src[min(k + e, K - 1)];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = k + e < K ? v[e] : (uint16_t)0;
-        }
-        return v;
+      auto row_of = [&](int q) __attribute__((always_inline)) {
+        return (q < NQA ? wave * NQA + q : wave * NQB + q - NQA) * RPK + lane / CH;
+      };
+      auto src = [&](int q) __attribute__((always_inline)) {
+        return q < NQA ? A0 + (int64_t)min(m0 + row_of(q), M - 1) * p.lda
+                       : B0 + (int64_t)min(n0 + row_of(q), N - 1) * p.ldb;
+      };
+      auto k_of = [&](int q) __attribute__((always_inline)) {
+        return kt0 + 8 * dl_swz(row_of(q), lane % CH);
       };
       u16x8_t v[NQA + NQB];
+      if (K >= 8) {
+        // a chunk that passes K as the row's last 8 elements, shifted down (M1500 N1000
+        // K130 12.3 us; 14.7 with a load per element)
+        typedef u16x8_t __attribute__((aligned(2))) u16x8_u;
 #pragma unroll
-      for (int q = 0; q < NQA + NQB; ++q) v[q] = get(q);
+        for (int q = 0; q < NQA + NQB; ++q) v[q] = *(const u16x8_u*)(src(q) + min(k_of(q), K - 8));
+#pragma unroll
+        for (int q = 0; q < NQA + NQB; ++q)
+          v[q] = __builtin_bit_cast(u16x8_t, shift_down(__builtin_bit_cast(u64x2_t, v[q]),
+                                                        2 * max(0, k_of(q) - (K - 8))));
+      } else {
+#pragma unroll
+        for (int q = 0; q < NQA + NQB; ++q)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const uint16_t x = src(q)[min(k_of(q) + e, K - 1)];
+            v[q][e] = k_of(q) + e < K ? x : (uint16_t)0;
+          }
+      }
 #pragma unroll
       for (int q = 0; q < NQA + NQB; ++q)
         *(u16x8_t*)(ts + (q < NQA ? (wave * NQA + q) * 512 : TA + (wave * NQB + q - NQA) * 512) +

@@ -23,7 +23,9 @@
 //
 // Addresses need only the element's alignment (a global dwordx4 load may start
 // at any 2-byte address), so odd K, row strides and bases run here as they
-// are; the last K % 64 (int8: 128) elements are read one by one by one wave.
+// are; the last K % 64 (int8: 128) elements are read by one wave, in chunks that end
+// with the row where they would pass it (element by element, int8 M33 N8192 K320
+// took 13.0 us, 6.3 so).
 #include <algorithm>
 
 #include "gemm_common.h"
@@ -53,9 +55,12 @@ __device__ __forceinline__ void rows_store(const GemmArgs& p, int64_t m, int64_t
     if constexpr (HAS_BIAS) x += p.beta * bb[e];
     v[e] = MfmaOp<T>::store(x);
   }
+  // (8 bytes at any element: element by element an odd row length, M17 N50257 K320,
+  // took 10.9 us, 9.4 so)
+  typedef u16x4_t __attribute__((aligned(2))) u16x4_u;
   uint16_t* dst = p.c + m * p.ldc + n;
-  if (n + 3 < p.N && (((uintptr_t)dst) & 7) == 0) {
-    *(u16x4_t*)dst = v;
+  if (n + 3 < p.N) {
+    *(u16x4_u*)dst = v;
   } else {
     for (int e = 0; e < 4 && n + e < p.N; ++e) dst[e] = v[e];
   }
@@ -63,8 +68,9 @@ __device__ __forceinline__ void rows_store(const GemmArgs& p, int64_t m, int64_t
 
 // I8: b is an int8 weight with fp32 scale per row (the int8 linear), its unit
 // 128 deep; a's 16 rows of a unit are then two tiles of 64.
+// Blocks of 16 waves keep to 64 registers, so that two share a CU.
 template <typename T, int MT, int RT, int NW, bool HAS_BIAS, bool SPLIT, bool I8>
-__global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* part, int64_t ldp) {
+__global__ __launch_bounds__(64 * NW, NW == 16 ? 8 : 1) void gemm_rows_kernel(GemmArgs p, float* part, int64_t ldp) {
   typedef typename MfmaOp<T>::vec vec;
   typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
   typedef u16x8 __attribute__((aligned(1))) u16x8_u1;
@@ -188,24 +194,47 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(GemmArgs p, float* p
   if (has_tail && wave == NW - 1) {
     const int64_t k0 = p.K / KU * KU;
     Unit u;
+    // k of the lane's first element of operand tile t
+    auto k_of = [&](int t) __attribute__((always_inline)) {
+      return k0 + (t < RT ? 16 / BE * (lane & 7) : 64 * ((t - RT) % XS) + 8 * (lane & 7));
+    };
+    auto src = [&](int t, int h) __attribute__((always_inline)) {
+      return base[t < RT ? 0 : 1] + off[t][h] + (t < RT ? k0 * BE : k0 * 2);
+    };
+    if (p.K * BE >= 16) {
+      // bytes of a lane's chunk that lie past the row
+      auto past = [&](int t) __attribute__((always_inline)) {
+        return (int)max((int64_t)0, (k_of(t) - p.K) * (t < RT ? BE : 2) + 16);
+      };
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const char* q = base[t < RT ? 0 : 1] + off[t][h] + (t < RT ? k0 * BE : k0 * 2);
-        // k of the lane's first element, elements per 16-bit word
-        const int64_t k = k0 + (t < RT ? 16 / BE * (lane & 7) : 64 * ((t - RT) % XS) + 8 * (lane & 7));
+        for (int h = 0; h < 2; ++h) u.v[t][h] = *(const u16x8_u*)(src(t, h) - past(t));
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if (I8 && t < RT) {
-            const uint16_t lo = k + 2 * e < p.K ? (uint8_t)q[2 * e] : 0;
-            const uint16_t hi = k + 2 * e + 1 < p.K ? (uint8_t)q[2 * e + 1] : 0;
-            u.v[t][h][e] = lo | (hi << 8);
-          } else {
-            u.v[t][h][e] = k + e < p.K ? ((const uint16_t*)q)[e] : (uint16_t)0;
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          u.v[t][h] = __builtin_bit_cast(u16x8, shift_down(__builtin_bit_cast(u64x2_t, u.v[t][h]), past(t)));
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const char* q = src(t, h);
+          const int64_t k = k_of(t);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            // (elements per 16-bit word: two of an int8 b)
+            if (I8 && t < RT) {
+              const uint16_t lo = k + 2 * e < p.K ? (uint8_t)q[2 * e] : 0;
+              const uint16_t hi = k + 2 * e + 1 < p.K ? (uint8_t)q[2 * e + 1] : 0;
+              u.v[t][h][e] = lo | (hi << 8);
+            } else {
+              u.v[t][h][e] = k + e < p.K ? ((const uint16_t*)q)[e] : (uint16_t)0;
+            }
           }
         }
-      }
+    }
     multiply(u);
   }
   // the waves' partial tiles reuse the staging tiles
@@ -272,8 +301,12 @@ mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
   return check_launch(what);
 }
 
-// Launch shape.  M <= 16: blocks of 16 weight rows; 16 waves (0-4 % faster up
-// to K = 8192), 8 beyond (M1 N4096 K11008: 20.0 us against 20.7).
+// Launch shape.  M <= 16: blocks of 16 weight rows and 8 waves, or 16 waves without
+// a bias for K = 4096 .. 8192 (M8 N4096 K8192 13.8 us against 14.8, N11008 K4096 16.4
+// against 16.8; K2048 9.8 against 9.3, and with a bias M8 N4096 K4096 6.8 against
+// 6.55).  Where such blocks go twice round the CUs and K <= 512, starting and adding
+// up the waves is most of the time: blocks of 64 rows and 4 waves (M8 N32000 K256
+// 5.4 us, 6.3 in 16-row blocks of 8 waves, 8.8 of 16).
 // M > 16: a's rows are read again by every block, and a CU takes in about
 // 55 KB/us whatever the source, so blocks of 64 weight rows (a quarter of that
 // traffic) wherever they number 128 or more (M64 N11008 K4096: 26 us against
@@ -284,8 +317,10 @@ mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
 template <typename T, int MT, bool HB>
 mi_status_t pick_mt(const GemmArgs& q, hipStream_t s, const char* what) {
   if constexpr (MT == 1) {
+    const bool wide = q.N >= 32 * (int64_t)cu_count();
+    if (wide && q.K <= 512) return launch<T, 1, 4, 4, HB, false>(q, 1, s, what);
     if constexpr (!HB)
-      if (q.K <= 8192) return launch<T, 1, 1, 16, HB, false>(q, 1, s, what);
+      if (q.K >= 4096 && q.K <= 8192) return launch<T, 1, 1, 16, HB, false>(q, 1, s, what);
     return launch<T, 1, 1, 8, HB, false>(q, 1, s, what);
   } else {
     const int64_t tiles = (q.N + 63) / 64;
@@ -299,7 +334,9 @@ mi_status_t pick_mt(const GemmArgs& q, hipStream_t s, const char* what) {
 // twice as much, but a unit's widening and four MFMAs per fragment favour small
 // blocks.  us: M8 N4096 K4224 10.8 -> 5.8, M15 N1920 K7123 106 -> 12.6, M24
 // N11008 K4224 28 -> 17 in blocks of 64 rows (19.5 in 16), M64 N4096 K4224 24 ->
-// 13 in 16 (16 sliced), M64 N4096 K8192 39 -> 19 sliced (22 in 16).
+// 13 in 16 (16 sliced), M64 N4096 K8192 39 -> 19 sliced (22 in 16).  Up to 16 rows,
+// 64-row blocks for K <= 512 from N = 40 x CUs (M8 N32000 K256 8.0 us in 16, 5.5 so;
+// M8 N8192 K512 4.9 and 5.2) and for K <= 1152 from 64 x CUs.
 template <typename T, int MT, bool HB>
 mi_status_t pick_mt8(const GemmArgs& q, hipStream_t s, const char* what) {
   if constexpr (MT > 1) {
@@ -307,6 +344,10 @@ mi_status_t pick_mt8(const GemmArgs& q, hipStream_t s, const char* what) {
     if (tiles >= 128) return launch<T, MT, 4, 4, HB, true>(q, 1, s, what);
     if (q.M * q.K >= (1 << 19))
       return launch<T, MT, 4, 4, HB, true>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
+  } else {
+    const int64_t cus = cu_count();
+    if ((q.N >= 40 * cus && q.K <= 512) || (q.N >= 64 * cus && q.K <= 1152))
+      return launch<T, MT, 4, 4, HB, true>(q, 1, s, what);
   }
   return launch<T, MT, 1, 8, HB, true>(q, 1, s, what);
 }
