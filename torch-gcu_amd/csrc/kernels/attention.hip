@@ -31,8 +31,9 @@
 // so that each of the 8 XCDs (which receive workgroups round robin) walks a
 // contiguous run of heads: a head's K/V is then read into one XCD's L2 while its
 // query tiles run there.  With a causal mask the tiles of a group of heads are
-// interleaved longest first, the group as large as its K and V fit the L2: head
-// by head, each head's longest tile started late and the last ones ran alone.
+// interleaved longest first, a group's K and V at most twice the L2 where two k/v
+// heads are: head by head, each head's longest tile started late and the last ones
+// ran alone.
 #include <algorithm>
 #include <cfloat>
 
@@ -555,14 +556,16 @@ extern "C" mi_status_t mi_flash_attention_fwd(const mi_tensor_t* out, const mi_t
   a.head_group = 1;
   if (a.causal && B * H % 8 == 0) {
     // the heads of one XCD in equal groups of at most 8 MB of K and V (twice its
-    // L2; groups of 4 and 8 MB time the same where both divide the heads).  us,
-    // head by head and so: [4, 32 (8 k/v), 1500, 128] 136 -> 115, [8, 32, 2048,
-    // 128] 405 -> 383, [4, 32, 2048, 128] 219 -> 197, [1, 32, 3195, 128] 136 ->
-    // 117, [8, 32, 512, 128] 52 -> 46
+    // L2; groups of 4 and 8 MB time the same where both divide the heads), two k/v
+    // heads where they are longer ([1, 32, 16384, 128] 2058 us, 2084 head by head; no
+    // difference with 8 k/v heads or at 32768).  us, head by head and so: [4, 32 (8
+    // k/v), 1500, 128] 136 -> 115, [8, 32, 2048, 128] 405 -> 383, [4, 32, 2048, 128]
+    // 219 -> 197, [1, 32, 3195, 128] 136 -> 117, [8, 32, 512, 128] 52 -> 46
     const int64_t heads = B * H / 8, kv = Sk * D * 4;
     const int64_t most = std::max<int64_t>(2, (8 << 20) / kv) * (H / Hk);
-    for (int64_t g = 1; g <= heads; ++g)
-      if (heads % g == 0 && g <= most) a.head_group = (int)g;
+    int64_t g = std::min(heads, most);
+    while (heads % g != 0) --g;
+    a.head_group = (int)g;
   }
   hipStream_t s = (hipStream_t)stream;
   mi_status_t st;
