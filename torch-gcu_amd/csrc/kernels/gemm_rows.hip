@@ -7,7 +7,7 @@
 // that of the stream plus about 3 us of launch, first latency and combine.
 // (The 32 x 64 tiles that ran here before made N / 64 blocks of two waves: N =
 // 4096 used a quarter of the CUs.)  us per call, before and now:
-//   M8 N4096 K4096 51 -> 8.4     M8 N11008 K4096 53 -> 18.4 (4.9 TB/s)
+//   M8 N4096 K4096 51 -> 8.4     M8 N11008 K4096 49 -> 16.7 (5.4 TB/s)
 //   M8 N32000 K4096 63 -> 45 (5.8 TB/s)   M1 N4096 K11008 128 -> 20
 //   M64 N11008 K4096 60 -> 26    M48 N4096 K11008 145 -> 25
 //
@@ -301,15 +301,18 @@ mi_status_t launch(const GemmArgs& q, int S, hipStream_t s, const char* what) {
   return check_launch(what);
 }
 
+// K slices for blocks of 64 weight rows that fill less than half the CUs
+int slices(int64_t tiles) { return (int)std::min<int64_t>(8, std::max<int64_t>(1, cu_count() / tiles)); }
+
 // Launch shape.  M <= 16: blocks of 16 weight rows and 8 waves, or 16 waves without
 // a bias for K = 4096 .. 8192 (M8 N4096 K8192 13.8 us against 14.8, N11008 K4096 16.4
-// against 16.8; K2048 9.8 against 9.3, and with a bias M8 N4096 K4096 6.8 against
-// 6.55).  Where such blocks go twice round the CUs and K <= 512, starting and adding
+// against 16.8; K2048 9.8 against 9.3, N128256 K4096 197 against 182, and with a bias
+// M8 N4096 K4096 6.8 against 6.55).  Where such blocks go twice round the CUs and K <= 512, starting and adding
 // up the waves is most of the time: blocks of 64 rows and 4 waves (M8 N32000 K256
 // 5.4 us, 6.3 in 16-row blocks of 8 waves, 8.8 of 16).
 // M > 16: a's rows are read again by every block, and a CU takes in about
 // 55 KB/us whatever the source, so blocks of 64 weight rows (a quarter of that
-// traffic) wherever they number 128 or more (M64 N11008 K4096: 26 us against
+// traffic) wherever they fill half the CUs (M64 N11008 K4096: 26 us against
 // 37).  With fewer, K is split over blocks when a is large enough to pay for
 // the combine, from M K = 2^18 (M48 N4096 K11008: 25 us against 31, M64 N1024
 // K9344: 15 against 26, M64 N4096 K4096: 14.4 against 14.5); below it blocks
@@ -320,13 +323,14 @@ mi_status_t pick_mt(const GemmArgs& q, hipStream_t s, const char* what) {
     const bool wide = q.N >= 32 * (int64_t)cu_count();
     if (wide && q.K <= 512) return launch<T, 1, 4, 4, HB, false>(q, 1, s, what);
     if constexpr (!HB)
-      if (q.K >= 4096 && q.K <= 8192) return launch<T, 1, 1, 16, HB, false>(q, 1, s, what);
+      if (q.K >= 4096 && q.K <= 8192 && q.N <= 128 * (int64_t)cu_count())
+        return launch<T, 1, 1, 16, HB, false>(q, 1, s, what);
     return launch<T, 1, 1, 8, HB, false>(q, 1, s, what);
   } else {
     const int64_t tiles = (q.N + 63) / 64;
-    if (tiles >= 128) return launch<T, MT, 4, 4, HB, false>(q, 1, s, what);
+    if (2 * tiles >= cu_count()) return launch<T, MT, 4, 4, HB, false>(q, 1, s, what);
     if (q.M * q.K < (1 << 18)) return launch<T, MT, 1, 8, HB, false>(q, 1, s, what);
-    return launch<T, MT, 4, 4, HB, false>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
+    return launch<T, MT, 4, 4, HB, false>(q, slices(tiles), s, what);
   }
 }
 
@@ -341,9 +345,9 @@ template <typename T, int MT, bool HB>
 mi_status_t pick_mt8(const GemmArgs& q, hipStream_t s, const char* what) {
   if constexpr (MT > 1) {
     const int64_t tiles = (q.N + 63) / 64;
-    if (tiles >= 128) return launch<T, MT, 4, 4, HB, true>(q, 1, s, what);
+    if (2 * tiles >= cu_count()) return launch<T, MT, 4, 4, HB, true>(q, 1, s, what);
     if (q.M * q.K >= (1 << 19))
-      return launch<T, MT, 4, 4, HB, true>(q, (int)std::min<int64_t>(8, 256 / tiles), s, what);
+      return launch<T, MT, 4, 4, HB, true>(q, slices(tiles), s, what);
   } else {
     const int64_t cus = cu_count();
     if ((q.N >= 40 * cus && q.K <= 512) || (q.N >= 64 * cus && q.K <= 1152))
