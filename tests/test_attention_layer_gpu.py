@@ -364,14 +364,11 @@ def test_attention_few_queries_long_cache(dtype, B, H, Hk, Sq, Sk, D, form):
     q, k, v = rn((B, H, Sq, D), 81, dtype), rn((B, Hk, Sk, D), 82, dtype), rn((B, Hk, Sk, D), 83, dtype)
     if form == "ramp":
         k = (k.float() * torch.linspace(0.2, 4.0, Sk)[None, None, :, None]).to(dtype)
-    if form == "negative_scale":
-        scale = -0.07
-        kk, vv = (t.repeat_interleave(H // Hk, 1).float().numpy() for t in (k, v))
-        ro, rl = npr.attention64(q.float().numpy(), kk, vv, False, scale)
-        ref, ref_lse = torch.from_numpy(ro).to(dtype), torch.from_numpy(rl).float()
-    else:
-        scale = None
-        ref, ref_lse = ref_attention(q, k, v, False)
+    scale = -0.07 if form == "negative_scale" else None
+    kk, vv = (t.repeat_interleave(H // Hk, 1).float().numpy() for t in (k, v))
+    ro, rl = npr.attention64(q.float().numpy(), kk, vv, False, scale)
+    ref_lse = torch.from_numpy(rl)
+    ref = torch.from_numpy(ro).to(dtype) if form == "negative_scale" else ref_attention(q, k, v, False)[0]
     if form == "heads_inner":
         dev = [t.transpose(1, 2).contiguous().cuda().transpose(1, 2) for t in (q, k, v)]
         out = torch.empty(B, Sq, H, D, dtype=dtype, device="cuda").transpose(1, 2)
@@ -381,7 +378,9 @@ def test_attention_few_queries_long_cache(dtype, B, H, Hk, Sq, Sk, D, form):
     lse = torch.empty(B, H, Sq, dtype=torch.float32, device="cuda")
     _abi.flash_attention_fwd(out, lse, *dev, False, scale)
     assert_close(out, ref, "bf16", f"few queries {B},{H},{Hk},{Sq},{Sk},{D} {form}")
-    assert (lse.cpu() - ref_lse).abs().max().item() < 2e-2 * max(1.0, ref_lse.abs().max().item())
+    # fp32 sums of positive terms: a lost tile of 32 keys or a lost split shows, a
+    # rounding of the scores (D products of up to 2^-24 of them, relative) does not
+    assert (lse.cpu().double() - ref_lse).abs().max().item() < 1e-3
 
 
 @pytest.mark.parametrize("B,H,Hk,S,D", [(1, 8, 8, 300, 128), (2, 8, 2, 260, 64), (4, 6, 3, 520, 128),
