@@ -8,8 +8,8 @@
 // the rows of one MFMA tile (up to 32; more rows take further tiles), and the
 // keys are split over blocks and, inside a block, over its four waves, which
 // never wait for each other: a wave streams its own 32-key tiles of K and V by
-// global_load_lds into a two-slot ring of its own (64 KiB in flight per CU) and
-// keeps its own running max, sum and O.  The four waves are merged through
+// global_load_lds into a two-slot ring of its own (a block's rings hold 128 KiB at
+// D = 128, 64 KiB at 64) and keeps its own running max, sum and O.  The four waves are merged through
 // LDS, the blocks' fp32 partials by flash_decode_combine_kernel in a fixed order.
 // MFMA layouts are the flash kernel's (S^T = K Q^T, P from registers,
 // O^T += V^T P^T with V^T by ds_read_b64_tr_b16), P rounded to the input type.
@@ -310,6 +310,9 @@ bool flash_decode(const AttnArgs& a, int64_t B, int64_t D, bool f16, hipStream_t
   // flash kernel and this one: 8 x 8 k/v heads of 4000 keys, G = 4: 96 / 30; 1 x
   // 32, 16000 keys, G = 1: 308 / 53; 12 x 16, 775 keys, G = 2, 8 queries: 33 /
   // 21; left out: 32 x 32, 512 keys, G = 1: 56 / 59; 4 x 8, 99 keys: 6.1 / 6.4.
+  // More than 64 rows stay with the flash kernel, which is the slower one for the few
+  // pairs of a long cache (4 k/v heads, 8000 keys, 72 rows: 156 / 18) and the faster
+  // one for many rows (8 x 8, 4000 keys, 256 rows: 90 / 149).
   DecodeArgs d{};
   d.rows = a.H / a.Hk * a.Sq;
   if (a.causal || d.rows > 64) return false;
@@ -318,7 +321,9 @@ bool flash_decode(const AttnArgs& a, int64_t B, int64_t D, bool f16, hipStream_t
   d.all_rows = B * a.H * a.Sq;
   const int64_t base = B * a.Hk * d.row_tiles;
   if (d.tiles < 8 || base > 0x7fffffff / 64) return false;
-  // one block per CU (128 KiB of LDS), every wave at least two tiles
+  // one block per CU (at D = 128 its LDS holds no more), every wave at least two
+  // tiles; pairs for more than half the CUs are not split (17 x 8 k/v heads of 4096
+  // keys, 136 blocks: 53 us, flash kernel 191)
   d.splits = (int)std::min<int64_t>(64, std::min<int64_t>(cu_count() / base, d.tiles / (2 * DNW)));
   if (d.splits < 2 && a.H == a.Hk) return false;
   Workspace ws;

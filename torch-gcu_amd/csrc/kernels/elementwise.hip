@@ -807,7 +807,8 @@ mi_status_t mi_copy(const mi_tensor_t* out, const mi_tensor_t* src, mi_stream_t 
       oc.ndim = nd - 1;  // the rows
       const int64_t pieces = (len + 15) / 16, total = it.numel / it.sizes[nd - 1] * pieces;
       if (total <= (int64_t)kBlock * 4 * 0x7fffffff) {
-        // four pieces a lane only where that leaves blocks for every CU
+        // four pieces a lane only where that leaves blocks for every CU (bf16
+        // [4, 100, 12, 64], its heads moved out: 4.3 us, 6.0 with four)
         if (total > (int64_t)kBlock * 4 * cu_count())
           hipLaunchKernelGGL(copy_rows_kernel<4>, dim3(ceil_div_u(total, kBlock * 4)), dim3(kBlock), 0,
                              stream, it.data[0], it.data[1], oc, esz, len, (uint32_t)pieces, total);

@@ -1217,9 +1217,13 @@ mi_status_t run_gemm(const mi_tensor_t* out, const mi_tensor_t* a, const mi_tens
   Workspace wa, wb, wc;
   Mat Bt = transposed(B);
   // Few rows: the weight stream kernels.  An int8 weight of whole 1 KiB slabs
-  // keeps int8_stream_kernel where its N / CUs rows per block are worth its 48-row
-  // slabs (M24 N11008 K4096 14.1 us against 16.4; M8 N4096 K4096 8.1 against 6.7,
-  // M64 N4096 K8192 39 against 19).  Asked of the operands as they are, and for
+  // keeps int8_stream_kernel from N = 32 x CUs.  Against the few-row kernel, us (N 8192
+  // .. 32000, K 1024 .. 11264): ahead up to 24 rows on N 9216 .. 11008 (M8 N11008 K4096
+  // 9.5 and 12.1, M24 13.9 and 16.1), even at N 8192 or 32 rows (M24 N8192 K4096 13.0
+  // and 15.0, M8 9.0 and 8.6), behind with more rows (M64 N11008 K8192 41 and 34) and
+  // where its 48-row slabs make an uneven last round (M24 N16384 K4096 24.6 and 17.2);
+  // below N = 32 x CUs behind (M8 N4096 K4096 8.1 and 6.7, M64 N4096 K8192 39 and 19).
+  // Asked of the operands as they are, and for
   // int8 of the dense copies where those were needed (M8 N4096 K4096, x at a column
   // stride of 2: 46 us on the large-M tiles, 9 so).
   auto few_rows = [&](const Mat& a, const Mat& bt, const Mat& c, mi_status_t* st) {

@@ -4,14 +4,15 @@
 //
 // What bounds the middle sizes: with one block or less per CU a K step costs its latency
 // until the ring holds enough steps in flight (two stages of 128 x 128 took
-// 0.80 us a step with 64 blocks, four stages 0.50), then the LDS: a wave's
-// 64 x 64 tile reads 16 KiB of fragments for 32 MFMAs.  So smaller tiles buy
+// 0.80 us a step with 64 blocks, four stages 0.50), then the matrix cores, with the
+// fragment reads behind them (M777 N4096 K11008: MFMA 0.68 of the busy cycles, LDS
+// 0.34; a wave's 64 x 64 tile reads 16 KiB for 32 MFMAs).  So smaller tiles buy
 // parallelism at more LDS traffic per MFMA, and K slices buy it at fp32
 // partial sums; which is cheaper depends on how many tiles there are.  The
 // register-staged 128 x 128 / 128 x 64 tiles that ran here had one step in
 // flight.  us, before and now (K-contiguous bf16 B):
 //   M128 N11008 K4096 60 -> 30      M256 N4096 K11008 140 -> 39
-//   M777 N4096 K11008 160 -> 75     M512 N1024 K1024  11 -> 6.2
+//   M777 N4096 K11008 161 -> 92     M512 N1024 K1024  11 -> 6.2
 //   M1024 N4096 K4096 58 -> 35      M2048 N4096 K4096 85 -> 55
 //   M4352 N4096 K4096 (272 tiles of 256 x 256, two rounds) 164 -> 144
 #include <algorithm>
@@ -173,9 +174,9 @@ mi_status_t launch_gemm_mid(const GemmArgs& q, int64_t batch, bool f16, bool has
 // shape of least cost.  Its bits are the unfused ops' only if those sum K in one
 // piece, so a product that launch_gemm_mid would slice is left to them (its
 // slices are also what makes it fast), and so is one whose products and
-// elementwise pass cost less.  us, unfused and fused: gate / up of 168 tokens
-// (N11008 K4096) 91 -> 62; on the 256 x 256 tiles alone before, 1496 tokens
-// (N5504 K2048, 258 tiles) 94 -> 76.
+// elementwise pass cost less.  us of kernel time
+// where only 256 x 256 tiles were fused, and now: gate / up of 168 tokens (N11008
+// K4096) 106 -> 46, of 1496 tokens (N5504 K2048, 258 tiles) 92 -> 84.
 bool launch_gemm_fused(const GemmArgs& q, bool silu, bool f16, hipStream_t s, const char* what,
                        mi_status_t* st) {
   const Pick plain = pick_shape(q, 1, true, 1);
