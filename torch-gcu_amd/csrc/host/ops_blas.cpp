@@ -2,7 +2,7 @@
 // (codegen/gcu_native_functions.yaml mm.out :452, addmm.out :205, bmm.out
 // :260, baddbmm.out :238, addmv.out :206; shape rules of
 // shape_inference/blas.cpp).  bf16 /
-// fp16 run on the MFMA kernel, fp32 on the VALU kernel; other dtypes take the
+// fp16 and fp32 run on the matrix instructions; other dtypes take the
 // CPU fallback as every unregistered op does.
 #include <ATen/ExpandUtils.h>
 #include <ATen/Operators.h>
