@@ -40,8 +40,9 @@ __device__ __forceinline__ int swz(int r, int c) {
   return c ^ (r & 3) ^ (((r >> 2) & 1) * 5) ^ ((r >> 1) & 4);
 }
 
-// out[m][n .. n + 3] = alpha * s (* scale[n]) + beta * bias, rounded once
-template <typename T, bool HAS_BIAS, bool I8>
+// out[m][n .. n + 3] = alpha * s (* scale[n]) + beta * bias, rounded once.  ANY: 8
+// bytes at any element (not in blocks of 16 waves: it costs them their 64 registers)
+template <typename T, bool HAS_BIAS, bool I8, bool ANY>
 __device__ __forceinline__ void rows_store(const GemmArgs& p, int64_t m, int64_t n, f32x4_t s) {
   f32x4_t bb = {}, sc = {1.f, 1.f, 1.f, 1.f};
   if constexpr (I8) sc = load_col4_t<T>(p.scale, MI_F32, n, 1, p.N, 0);
@@ -59,7 +60,7 @@ __device__ __forceinline__ void rows_store(const GemmArgs& p, int64_t m, int64_t
   // took 10.9 us, 9.4 so)
   typedef u16x4_t __attribute__((aligned(2))) u16x4_u;
   uint16_t* dst = p.c + m * p.ldc + n;
-  if (n + 3 < p.N) {
+  if (n + 3 < p.N && (ANY || (((uintptr_t)dst) & 7) == 0)) {
     *(u16x4_u*)dst = v;
   } else {
     for (int e = 0; e < 4 && n + e < p.N; ++e) dst[e] = v[e];
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(64 * NW, NW == 16 ? 8 : 1) void gemm_rows_kernel(Ge
       *(f32x4_t*)(part + ((int64_t)blockIdx.y * p.M + m) * ldp + n) = s;
       continue;
     }
-    rows_store<T, HAS_BIAS, I8>(p, m, n, s);
+    rows_store<T, HAS_BIAS, I8, NW != 16>(p, m, n, s);
   }
 }
 
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(256) void rows_combine_kernel(GemmArgs p, const flo
   f32x4_t s = *(const f32x4_t*)src;
 #pragma unroll 8
   for (int i = 1; i < S; ++i) s += *(const f32x4_t*)(src + i * p.M * ldp);
-  rows_store<T, HAS_BIAS, I8>(p, m, n, s);
+  rows_store<T, HAS_BIAS, I8, true>(p, m, n, s);
 }
 
 template <typename T, int MT, int RT, int NW, bool HB, bool I8>
@@ -306,7 +307,7 @@ int slices(int64_t tiles) { return (int)std::min<int64_t>(8, std::max<int64_t>(1
 
 // Launch shape.  M <= 16: blocks of 16 weight rows and 8 waves, or 16 waves without
 // a bias for K = 4096 .. 8192 (M8 N4096 K8192 13.8 us against 14.8, N11008 K4096 16.4
-// against 16.8; K2048 9.8 against 9.3, N128256 K4096 197 against 182, and with a bias
+// against 16.8; K2048 9.8 against 9.3, N128256 K4096 183 against 182, and with a bias
 // M8 N4096 K4096 6.8 against 6.55).  Where such blocks go twice round the CUs and K <= 512, starting and adding
 // up the waves is most of the time: blocks of 64 rows and 4 waves (M8 N32000 K256
 // 5.4 us, 6.3 in 16-row blocks of 8 waves, 8.8 of 16).
